@@ -707,3 +707,53 @@ def test_mod_select_parity(dev, B, S, keep, ties):
     om = np.full(B * S, -1)
     om[exp_rows] = np.arange(B * keep)
     assert np.array_equal(out.out_map.cpu().numpy(), om)
+
+
+# ------------------------------------------------------------------ full-tile loop
+@pytest.mark.parametrize("path,d", [("rows", 64), ("rows", 128), ("rows", 192), ("rows", 320), ("rscale", 128),
+                                    ("rscale", 256), ("save_gu", 128), ("save_gu", 192), ("fp8", 128), ("fp8", 256),
+                                    ("fp8", 384)])
+def test_full_tile_loop(dev, path, d):
+    """Several full tiles per workgroup (more than two tiles per CU) with one, two, three
+    and more K-steps (d 64 per step, fp8 128), experts of 0, 1, 33, 64, 65 and many rows:
+    the gate/up product against fp32 matmuls of the same operands (fp8: the dequantised
+    ones).  A wrong stage, row lookup or scale set of a following tile gives an error of
+    order 1; rounding h to bf16 gives 2^-9 at most per value (bar 4e-3 rel-L2)."""
+    F = 256
+    n_cu = torch.cuda.get_device_properties(dev).multi_processor_count
+    counts = [1, 0, 33, 64, 65, 256, 256 * (n_cu // 3) + 17, 256 * (n_cu // 2) + 129]
+    E, A = len(counts), sum(counts)
+    off_l = np.concatenate([[0], np.cumsum(counts)])
+    off = torch.tensor(off_l, dtype=torch.int32, device=dev)
+    g = torch.Generator(device=dev).manual_seed(d)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    T = 4096
+    x = bf16(rnd(T, d))
+    w1, w2, w3 = (bf16(rnd(*s) * s[1] ** -0.5) for s in ((E, d, F), (E, d, F), (E, F, d)))
+    rt = torch.randint(0, T, (A,), generator=g, device=dev, dtype=torch.int32)
+    pw = ops.pack_weights(w1, w2, w3, fp8=path == "fp8")
+    rs = torch.rand(T, generator=g, device=dev) + 0.5
+    gu = None
+    if path == "fp8":
+        xq, xsc = ops.gather_rows(x, rt, A, fp8=True)
+        h = ops.gemm_gate_up(xq, xsc, off, pw, A)
+        xr = ops.dequant_rows_fp8(xq, torch.ones_like(xsc)).float() * xsc[:, None]
+        # codes are exact in bf16; scale the columns like the packing (amax / 448)
+        w1, w2 = (ops.fake_quant_cols_e4m3(w) for w in (w1, w2))
+    else:
+        h = ops.gemm_gate_up_rows(x, None, rt, off, pw, A, save_gu=path == "save_gu",
+                                  rscale=rs if path == "rscale" else None)
+        if path == "save_gu":
+            h, gu = h
+        xr = x[rt.long()].float() * (rs[rt.long(), None] if path == "rscale" else 1.0)
+    for e in range(E):
+        s, t = int(off_l[e]), int(off_l[e + 1])
+        if s == t:
+            continue
+        gg, uu = xr[s:t] @ w1[e].float(), xr[s:t] @ w2[e].float()
+        ref = torch.nn.functional.silu(gg) * uu
+        rel = lambda a, b: float((a.float() - b).norm() / b.norm())
+        assert rel(h[s:t, :F], ref) <= 4e-3, (path, d, e, counts[e])
+        if gu is not None:
+            packed = torch.cat([gg[:, :128], uu[:, :128], gg[:, 128:], uu[:, 128:]], 1)
+            assert rel(gu[s:t], packed) <= 4e-3, (path, d, e, counts[e])
