@@ -14,9 +14,11 @@ int launch_gemm(bool gate_up, bool fp8, const void* A, const float* a_scale, con
                 int n_tiles, hipStream_t s, void* C2 = nullptr, void* gu_out = nullptr) {
   const int eb = fp8 ? 1 : 2;
   const int64_t slots = kmoe::ceil_div<int64_t>(max_rows, BM) + E;
-  // one workgroup per CU, looping over its tiles (as many as there can be narrow tiles, if fewer)
+  // every tile of the worst-case slot count, plus one narrow tile per resident
+  // workgroup for the split tail (e4m3: one workgroup per CU and the
+  // narrow tiles, or with a single K-step every tile in halves)
   const int n_cu = kmoe::cu_count();
-  const int64_t blocks = std::min<int64_t>(4 * slots * n_tiles, n_cu);
+  const int64_t blocks = !fp8 ? slots * n_tiles + n_cu : K >= 2 * KB ? 2 * n_cu : 2 * slots * n_tiles;
   if (blocks > 0x7fffffff) {
     kmoe::set_error("kmoe gemm: grid too large");
     return KMOE_ERR_SHAPE;

@@ -22,12 +22,13 @@
 // groups, fragments double buffered.  One barrier per step.
 // The MFMAs take the B fragment as their first operand, so each lane accumulates
 // runs of four consecutive output columns of one row; the epilogue packs them to
-// 8-byte bf16 runs in registers, merges them across lanes to 16 bytes and stores whole
-// 128-byte row segments (narrow tiles: through LDS).
+// 8-byte bf16 runs in registers, stages the tile through LDS and writes it with
+// 16-byte row stores (full e4m3 tiles: merged across lanes and stored from registers).
 //
 // Ragged groups: every row tile ("slot") of every expert is enumerated from the
-// device-resident offsets; the grid is one workgroup per CU, each looping over its tiles
-// (gemm_full_tiles).  No host sync.
+// device-resident offsets; the grid is sized for the worst case
+// (ceil(max_rows/256) + E slots) and workgroups without a tile exit (full e4m3 tiles: one
+// workgroup per CU loops over its tiles).  No host sync.
 // Tile order is XCD-aware: workgroups are dispatched round-robin over the 8 XCDs,
 // so consecutive ids of one XCD are given 32-tile super-blocks of 4 slots x 8
 // column tiles, which then share their A and B K-slices in that XCD's L2.
@@ -334,17 +335,29 @@ __device__ __forceinline__ void store_staged(const uint8_t* lds, int tid, int m0
 // between C and C2 (the gate and up halves of a w13-ordered tile); fp32 to Cf.
 constexpr int OUT_BF16 = 0, OUT_SPLIT = 1, OUT_F32 = 2;
 
-// One narrow output tile: rows [m0, min(m0 + 256, m_end)) of expert e against part q (64 WNB
-// B rows) of full column tile nt, for the split tail of a launch and single-step products.
-// The template flags are those of gemm_full_tiles.
-template <bool GATE_UP, bool FP8, bool GATHER, int WNB, bool SAVE_GU, bool RSCALE>
-__device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int e, int m0, int m_end, int nt,
-                                            int q) {
-  static_assert(WNB == 2 || WNB == 1, "tile width");
-  // bf16: 16x16x32 MFMAs, 16-row A and B blocks (MA x NBB per wave); fp8: 32x32x64, 32-row
-  // blocks
+// One output tile: rows [m0, min(m0 + 256, m_end)) of expert e against B rows of
+// full column tile nt (narrow part q when WNB < 4).
+// FP8: A/B bytes are e4m3; a_scale per A row, b_scale per B row (global row index).
+// GATHER: A is the unpermuted activation matrix and permuted row r is its row
+// row_index[row_token[r]] (row_token[r] without row_index): the dispatch gather is
+// fused into the A loads.
+// RSCALE (bf16 gathered gate/up tiles): a_scale[row_token[r]] scales row r's gate and
+// up values before the SiLU (the per-token RMSNorm scale of x: the norm weight is
+// folded into the packed w1 / w2 rows, and a per-row scale commutes with the product).
+// NMA: the row blocks of this wave that hold rows of the expert.  A wave's 128 rows
+// are 4 blocks of 32; a slot's last tile is often partly empty, and its waves then
+// run with NMA < 4 (the first NMA blocks), which skips the other blocks' fragment
+// reads, MFMAs and epilogue (their accumulators stay 0 and are never stored).  The
+// waves of a workgroup may differ in NMA: loads, LDS writes and barriers are the same.
+template <bool GATE_UP, bool FP8, bool GATHER, int WNB, bool SAVE_GU = false, bool RSCALE = false, int NMA = 4>
+__device__ __forceinline__ void gemm_tile(const GemmArgs& g, uint8_t* lds, int e, int m0, int m_end, int nt,
+                                          int q) {
+  static_assert(WNB == 4 || WNB == 2 || WNB == 1, "tile width");
+  // bf16: 16x16x32 MFMAs, 16-row A and B blocks (MA x NBB per wave, NAB of them holding
+  // rows); fp8: 32x32x64, 32-row blocks
   constexpr bool M16 = !FP8;
   constexpr int MA = M16 ? 8 : 4;
+  constexpr int NAB = M16 ? 2 * NMA : NMA;
   constexpr int NBB = M16 ? 2 * WNB : WNB;
   using Acc = std::conditional_t<M16, f32x4_t, f32x16_t>;
   constexpr int ACCN = M16 ? 4 : 16;
@@ -395,7 +408,7 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
   // there: the LDS write of a block is one contiguous, conflict-free 1 KiB.  A rows
   // past the expert's last row read as zeros (their results are never stored).
   const int rsub = lane / CPR, pc = lane % CPR;
-  uint32_t a_off[BLK_PER_WAVE], b_off[BLK_B];
+  uint32_t a_off[BLK_PER_WAVE], b_off[8];
   const int a_last = m_end - 1 - m0;
   int ra[BLK_PER_WAVE];
 #pragma unroll
@@ -430,7 +443,7 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
     const uint32_t chunk = (uint32_t)(pc ^ ((tr >> 1) & (CPR - 1))) << 4;
     b_off[qb] = (uint32_t)b_packed_row<GATE_UP, WNB>(tr, q) * (uint32_t)g.ldb_bytes + chunk;
   }
-  i32x4_t stg[NBLK];  // one step of this wave's tile data: A blocks, then B blocks
+  i32x4_t stg[16];  // one step of this wave's tile data: A blocks, then B blocks
   // block qq: global -> registers (K-step kt, clamped to the last step)
   auto load_block = [&](int qq, int kt) {
     const int ks = kt < nk ? kt : nk - 1;
@@ -448,19 +461,21 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
   Frag<FP8> fa[2][MA], fb[2][NBB];
   const int r16 = lane & 15, lq = lane >> 4;
   auto rd = [&](int st, int i, Frag<FP8> (&a)[MA], Frag<FP8> (&b)[NBB]) {
-    const uint8_t* la = la_buf(st);
-    const uint8_t* lb = lb_buf(st);
-    if constexpr (M16) {
+    if constexpr (NMA > 0) {
+      const uint8_t* la = la_buf(st);
+      const uint8_t* lb = lb_buf(st);
+      if constexpr (M16) {
 #pragma unroll
-      for (int j = 0; j < NBB; ++j)
-        read_frag16(lb, b_lds_row<GATE_UP, WNB>(wn, j >> 1, 16 * (j & 1) + r16), i, lq, b[j]);
+        for (int j = 0; j < NBB; ++j)
+          read_frag16(lb, b_lds_row<GATE_UP, WNB>(wn, j >> 1, 16 * (j & 1) + r16), i, lq, b[j]);
 #pragma unroll
-      for (int mi = 0; mi < MA; ++mi) read_frag16(la, wm * 128 + mi * 16 + r16, i, lq, a[mi]);
-    } else {
+        for (int mi = 0; mi < NAB; ++mi) read_frag16(la, wm * 128 + mi * 16 + r16, i, lq, a[mi]);
+      } else {
 #pragma unroll
-      for (int mi = 0; mi < MA; ++mi) read_frag<FP8>(la, wm * 128 + mi * 32 + lr, i, lh, a[mi]);
+        for (int mi = 0; mi < NMA; ++mi) read_frag<FP8>(la, wm * 128 + mi * 32 + lr, i, lh, a[mi]);
 #pragma unroll
-      for (int j = 0; j < WNB; ++j) read_frag<FP8>(lb, b_lds_row<GATE_UP, WNB>(wn, j, lr), i, lh, b[j]);
+        for (int j = 0; j < WNB; ++j) read_frag<FP8>(lb, b_lds_row<GATE_UP, WNB>(wn, j, lr), i, lh, b[j]);
+      }
     }
   };
   auto mma1 = [&](Acc& c, const Frag<FP8>& b, const Frag<FP8>& a) {
@@ -471,7 +486,7 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
   };
   auto mma = [&](const Frag<FP8> (&a)[MA], const Frag<FP8> (&b)[NBB]) {
 #pragma unroll
-    for (int mi = 0; mi < MA; ++mi)
+    for (int mi = 0; mi < NAB; ++mi)
 #pragma unroll
       for (int j = 0; j < NBB; ++j) mma1(acc[mi][j], b[j], a[mi]);
   };
@@ -487,14 +502,14 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
   // tile data.  Those blocks are written into stage (kt+1)%2 (which every wave
   // stopped reading at step kt-1's barrier) over the substeps, each block reloaded
   // with step kt+2's data right after its write, so a load has a whole step to land
-  // and the LDS write traffic is spread (half in each
-  // substep).  In the last substep, after most of
+  // and the LDS write traffic is spread (bf16: about 6/5/5 sixteenths of the blocks
+  // in substeps 0-2; fp8: half in each substep).  In the last substep, after most of
   // its MFMAs, the wave waits for its LDS writes and reads, then one barrier publishes
   // stage kt+1, whose first fragments are read under the last few MFMAs.  Register
   // dependencies give the vmcnt waits; the scheduling groups interleave the LDS and
   // memory operations with the MFMAs, fragment reads first.
-  constexpr int RD = (FP8 ? 2 : 1) * (MA + NBB);  // LDS reads of a substep's fragments
-  constexpr int NMS = MA * NBB;                   // MFMAs per substep
+  constexpr int RD = NMA > 0 ? (FP8 ? 2 : 1) * (NAB + NBB) : 0;  // LDS reads of a substep's fragments
+  constexpr int NMS = NAB * NBB;                                    // MFMAs per substep
   for (int qq = 0; qq < NBLK; ++qq) load_block(qq, 0);
   for (int qq = 0; qq < NBLK; ++qq) write_block(qq, 0);
   for (int qq = 0; qq < NBLK; ++qq) load_block(qq, 1);
@@ -502,9 +517,24 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
   barrier_nofence();
   if constexpr (!M16) rd(0, 0, fa[0], fb[0]);
 
-  // bf16: one MFMA at a time in program order, as gemm_full_tiles' step16 (whose comment
-  // has the reasons), the reads, block writes and reloads spread evenly.
-  constexpr int GB = NMS - 1 - (NBB + MA < NMS - 1 ? NBB + MA : NMS - 1);  // substep 1: barrier after MFMA GB
+  // bf16 (16x16 blocks): the K loop is emitted in program order, one MFMA at a time,
+  // each followed by the LDS reads, block writes or reloads assigned to it and fenced
+  // with sched_barrier.  (With scheduling groups the scheduler may take the MFMAs out of
+  // order, and the register allocator then stops tying each MFMA's accumulator input to
+  // its output: hundreds of accumulator copies per K-step.)  A 16x16x32 MFMA keeps the
+  // matrix pipe 16 cycles, about what a 1 KiB LDS block write takes to issue, so the
+  // schedule gives each MFMA at most one LDS or memory instruction where it can.
+  // Substep i uses B fragment set fb[i] and the one A set fa[0]; MFMAs go row block by
+  // row block.  Substep 0 reads substep 1's B fragments into fb[1] and each row block's
+  // next A fragment right after that row block's last MFMA (an A ring: no second A set).
+  // Substep 1 meets the other waves at the barrier that publishes stage nxt after MFMA
+  // GB, then reads that stage's substep-0 fragments (B0, A0, B1, ..., each A after its
+  // row block's last MFMA).  The block writes into stage nxt and the reloads of step kt+2
+  // go over substep 0 and the part of substep 1 before the barrier, each reload a few
+  // MFMAs after the write that frees its registers.
+  constexpr bool FULL16 = NMS == 64 && NBB == 8 && NAB == 8 && NBLK == 16;
+  constexpr int NR16 = NMS > 0 ? ((NBB + NAB) < NMS - 1 ? NBB + NAB : NMS - 1) : 0;
+  constexpr int GB = FULL16 ? 31 : NMS - 1 - NR16;  // substep 1: the barrier follows MFMA GB
   constexpr int H0 = NBLK / 2;                      // block writes in substep 0 (the rest in substep 1)
   auto rdB16 = [&](int st, int i, int j, Frag<FP8>& b) {
     if constexpr (M16) read_frag16(lb_buf(st), b_lds_row<GATE_UP, WNB>(wn, j >> 1, 16 * (j & 1) + r16), i, lq, b);
@@ -517,18 +547,38 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
     constexpr bool LAST = decltype(last_tag)::value;
     const int cur = kt & 1, nxt = cur ^ 1;
     constexpr int NW = LAST ? 0 : (i == 0 ? H0 : NBLK - H0), QB = i == 0 ? 0 : H0;
+    if constexpr (NMS == 0) {
+      // a wave without rows: only its share of the tile loads and the barrier
+      if constexpr (NW > 0) {
+        static_for<0, NW>([&](auto wc) {
+          write_block(QB + decltype(wc)::value, nxt);
+          load_block(QB + decltype(wc)::value, kt + 2);
+        });
+      }
+      if constexpr (i == 1 && !LAST) {
+        wait_lgkmcnt0();
+        barrier_nofence();
+      }
+      return;
+    }
     // MFMA after which block write w / its reload go (w < NW; NW1 keeps the division
     // defined in the instantiations without block writes)
     constexpr int NW1 = NW > 0 ? NW : 1;
     constexpr auto w_at = [](int w) constexpr {
+      if (FULL16) return i == 0 ? 16 + 6 * w : 4 * w;
+      const int span = i == 0 ? NMS - 2 : GB - 2;
+      return span > 0 ? 1 + (w * span) / NW1 : 0;
+    };
+    constexpr auto l_at = [](int w) constexpr {
+      if (FULL16) return i == 0 ? 18 + 6 * w : 4 * w + 2;
       const int span = i == 0 ? NMS - 2 : GB - 2;
       return span > 0 ? 1 + (w * span) / NW1 : 0;
     };
     // substep 0: MFMA after which next-substep read B_j / A_mi goes
-    constexpr auto b0_at = [](int j) constexpr { return j < NMS ? j : NMS - 1; };
+    constexpr auto b0_at = [](int j) constexpr { return FULL16 ? 2 * j : (j < NMS ? j : NMS - 1); };
     // substep 1: post-barrier read k (0: B0, 1: A0, 2 ..: B1 .. B_{NBB-1}, then A1 ..)
     constexpr auto post_at = [](int k, int kind, int idx) constexpr {
-      const int e0 = GB + 1 + k;
+      const int e0 = GB + 1 + (FULL16 ? 2 * k + 1 : k);
       const int e1 = kind == 1 ? idx * NBB + NBB - 1 : 0;
       const int at = e0 > e1 ? e0 : e1;
       return at < NMS - 1 ? at : NMS - 1;
@@ -545,7 +595,7 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
       });
       static_for<0, NW>([&](auto wc) {
         constexpr int w = decltype(wc)::value;
-        if constexpr (w_at(w) == g) load_block(QB + w, kt + 2);
+        if constexpr (l_at(w) == g) load_block(QB + w, kt + 2);
       });
       if constexpr (i == 0) {
         static_for<0, NBB>([&](auto jc) {
@@ -558,7 +608,7 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
           wait_lgkmcnt0();
           barrier_nofence();
         }
-        static_for<0, NBB + MA>([&](auto kc) {
+        static_for<0, NBB + NAB>([&](auto kc) {
           constexpr int k = decltype(kc)::value;
           constexpr int kind = k == 0 ? 0 : k == 1 ? 1 : k < NBB + 1 ? 0 : 1;
           constexpr int idx = k == 0 ? 0 : k == 1 ? 0 : k < NBB + 1 ? k - 1 : k - NBB;
@@ -578,10 +628,12 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
     sub16(kt, std::integral_constant<int, 1>{}, last_tag);
   };
   if constexpr (M16) {
+    if constexpr (NMA > 0) {
 #pragma unroll
-    for (int j = 0; j < NBB; ++j) rdB16(0, 0, j, fb[0][j]);
+      for (int j = 0; j < NBB; ++j) rdB16(0, 0, j, fb[0][j]);
 #pragma unroll
-    for (int mi = 0; mi < MA; ++mi) rdA16(0, 0, mi);
+      for (int mi = 0; mi < NAB; ++mi) rdA16(0, 0, mi);
+    }
   }
   auto step = [&](int kt, auto last_tag) {
     if constexpr (M16) {
@@ -593,10 +645,13 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
     static_for<0, NSUB>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
       constexpr int bi = i & 1;
-      // blocks [q0, q1) are written and reloaded in this substep, the last substep's before
-      // its barrier (all in substep 0 crowded the LDS queue with that substep's fragment
-      // reads: 3% slower)
-      constexpr int q0 = i * NBLK / NSUB, q1 = (i + 1) * NBLK / NSUB;
+      // blocks [q0, q1) are written and reloaded in this substep.  bf16 (4 substeps):
+      // about 6/5/5 sixteenths in substeps 0-2.  fp8 (2 substeps): half in each, the
+      // last substep's before its barrier (all in substep 0 crowded the LDS queue with
+      // that substep's fragment reads: 3% slower).
+      constexpr int C1 = (NBLK * 6 + 8) / 16, C2 = (NBLK * 11 + 8) / 16;
+      constexpr int q0 = NSUB == 4 ? (i == 0 ? 0 : i == 1 ? C1 : i == 2 ? C2 : NBLK) : i * NBLK / NSUB;
+      constexpr int q1 = NSUB == 4 ? (i == 0 ? C1 : i == 1 ? C2 : NBLK) : (i + 1) * NBLK / NSUB;
       constexpr int nq = LAST ? 0 : q1 - q0;
       constexpr bool RDN = i + 1 < NSUB || !LAST;
       // next substep's fragments first: they are on the MFMA critical path
@@ -706,7 +761,7 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
     constexpr int NJ16 = GATE_UP ? NBB / 2 : NBB;
     uint8_t* const wb16 = lds + (wm * 128 + r16) * OSTR + (wn * (NC / 2) + 4 * lq) * 2;
 #pragma unroll
-    for (int mi = 0; mi < MA; ++mi) {
+    for (int mi = 0; mi < NAB; ++mi) {
       if constexpr (RSCALE) sar = sa_l[wm * 128 + mi * 16 + r16];
 #pragma unroll
       for (int jo = 0; jo < NJ16; ++jo) {
@@ -732,6 +787,7 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
     uint8_t* const wbase = lds + (wm * 128 + lr) * OSTR + (wn * (NC / 2) + 4 * lh) * 2;
 #pragma unroll
     for (int mi = 0; mi < 4; ++mi) {
+      if (mi >= NMA) break;  // rows past the expert's end: never stored
       if constexpr (FP8 || RSCALE) sar = sa_l[wm * 128 + mi * 32 + lr];
 #pragma unroll
       for (int jo = 0; jo < NJ; ++jo)
@@ -757,7 +813,7 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
     if constexpr (M16) {
       uint8_t* const wb2 = lds + (wm * 128 + r16) * OSTR2 + 4 * lq * 2;
 #pragma unroll
-      for (int mi = 0; mi < MA; ++mi)
+      for (int mi = 0; mi < NAB; ++mi)
 #pragma unroll
         for (int j = 0; j < NBB; ++j) {
           const int col = b_lds_row<true, WNB>(wn, j >> 1, 16 * (j & 1));
@@ -768,6 +824,7 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
       uint8_t* const wb2 = lds + (wm * 128 + lr) * OSTR2 + 4 * lh * 2;
 #pragma unroll
       for (int mi = 0; mi < 4; ++mi) {
+        if (mi >= NMA) break;
         if constexpr (FP8) sar = sa_l[wm * 128 + mi * 32 + lr];
 #pragma unroll
         for (int j = 0; j < WNB; ++j) {
@@ -790,34 +847,13 @@ __device__ __forceinline__ void narrow_tile(const GemmArgs& g, uint8_t* lds, int
   }
 }
 
-
-// Lane groups of 16 hold runs of four output columns (two dwords of bf16) of two adjacent
-// 16-column blocks x, y: after the row swaps a lane holds eight consecutive columns of one
-// of them (block lq & 1, columns 8 (lq / 2) .. + 7, lq = lane / 16), one 16-byte store.
-__device__ __forceinline__ i32x4_t merge16(i32x2_t x, i32x2_t y) {
-  const auto a = __builtin_amdgcn_permlane16_swap((unsigned)x[0], (unsigned)y[0], false, false);
-  const auto b = __builtin_amdgcn_permlane16_swap((unsigned)x[1], (unsigned)y[1], false, false);
-  return i32x4_t{(int)a[0], (int)b[0], (int)a[1], (int)b[1]};
-}
-// The same for 32x32 blocks, whose half waves hold runs 8c + 4 (lane / 32): x is run c, y
-// run c + 1; a lane ends with the eight columns of run c + lane / 32.
+// The half waves of a 32x32 block hold runs of four output columns 8c + 4 (lane / 32) (two
+// dwords of bf16): from runs x = c and y = c + 1 a lane gets the eight consecutive columns
+// of run c + lane / 32, one 16-byte store.
 __device__ __forceinline__ i32x4_t merge32(i32x2_t x, i32x2_t y) {
   const auto a = __builtin_amdgcn_permlane32_swap((unsigned)x[0], (unsigned)y[0], false, false);
   const auto b = __builtin_amdgcn_permlane32_swap((unsigned)x[1], (unsigned)y[1], false, false);
   return i32x4_t{(int)a[0], (int)b[0], (int)a[1], (int)b[1]};
-}
-// Two 16-byte pieces p, q of a lane's row (lane % 16; q 64 bytes after p) exchanged with the
-// row eight below or above, so that a store covers eight whole 128-byte row segments and
-// not sixteen halves: first p of rows 0 .. 7 (lanes r) and their q (lanes r + 8), then
-// the same of rows 8 .. 15.
-__device__ __forceinline__ void swap_halves(i32x4_t& p, i32x4_t& q, bool low) {
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int give = low ? q[c] : p[c];
-    const int got = __builtin_amdgcn_update_dpp(0, give, 0x128, 0xF, 0xF, false);  // row_ror:8
-    p[c] = low ? p[c] : got;
-    q[c] = low ? got : q[c];
-  }
 }
 __device__ __forceinline__ i32x2_t pack4_bf16(float a, float b, float c, float d) {
   const uint32_t lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));
@@ -826,52 +862,37 @@ __device__ __forceinline__ i32x2_t pack4_bf16(float a, float b, float c, float d
 }
 
 // LDS of the full-tile loop behind its stages: the experts' slot table (lo, hi, inclusive
-// slot count of each), the next tile's row tokens, and two sets of A-row and B-row scales.
+// slot count of each) and two sets of A-row and B-row scales.
 constexpr int FT_SLOTS = NST * 2 * TB;
-constexpr int FT_TOK = FT_SLOTS + 3 * 64 * 4;
-constexpr int FT_SCALE = FT_TOK + BM * 4;
+constexpr int FT_SCALE = FT_SLOTS + 1024;
 constexpr int FT_LDS = FT_SCALE + 2 * 2 * BM * 4;
 static_assert(FT_LDS <= GEMM_LDS, "LDS of the full-tile loop");
 
-// The full 256 x 256 tiles of a workgroup: tiles L = blockIdx.x, + gridDim.x, .. < n_full,
-// in one continuous K pipeline.  The last two K-steps of a tile load the next tile's first
-// two (its rows and scales were looked up at the start of the tile), so the next tile
+// The full 256 x 256 tiles of a workgroup of an e4m3 product: tiles L = blockIdx.x, + n_cu,
+// .. < n_full, in one continuous K pipeline.  The last two K-steps of a tile load the next
+// tile's first two (its scales were looked up at the start of the tile), so the next tile
 // starts with its first stage in LDS and its second step in flight, and the epilogue
-// stores straight from registers.  One workgroup fills a CU (128 KiB of stages, 500
-// registers), so whatever runs between two tiles leaves its matrix cores idle.  Against
-// one workgroup per tile with stores staged through LDS: gate/up of 32768 rows, d 2048,
-// F 2816 660 -> 637 us; the e4m3 layer at 8192 tokens 375 -> 358 us.  What is left between
-// two tiles (per tile at K = 2048, of 56 us): about 6 us of stores (2.5 us on an otherwise
-// idle chip; whole 128-byte rows, non-temporal stores and staggered workgroups measured
-// the same) and 1.5 us of packing; the K loop runs at 0.73 of the matrix rate uncontended.
-// Needs at least two K-steps.
-// NMA (4, 2, 1 or 0, per tile and wave): the wave's 32-row blocks that hold rows of the
+// stores straight from registers.  One workgroup fills a CU (128 KiB of stages, 512
+// registers), so whatever runs between two tiles leaves its matrix cores idle, and an
+// e4m3 tile has half the K-steps of a bf16 one: the layer of 8192 tokens (6144 kept), d
+// 2048, F 2816 375 -> 358 us against one workgroup per tile.  (bf16 tiles the same way: 1045
+// -> 1025 us at 16384 tokens, eleven rounds, but 2% slower at one to three rounds; they
+// stay one workgroup per tile.)  Needs at least two K-steps.
+// NMA (4, 2 or 0, per tile and wave): the wave's 32-row blocks that hold rows of the
 // expert; the others' fragment reads, MFMAs and stores are skipped.  The waves of a
 // workgroup may differ in NMA: loads, LDS writes and barriers are the same.
-// FP8: A/B bytes are e4m3; a_scale per A row, b_scale per B row (global row index).
-// GATHER: A is the unpermuted activation matrix and permuted row r is its row
-// row_index[row_token[r]] (row_token[r] without row_index): the dispatch gather is
-// fused into the A loads.
-// RSCALE (bf16 gathered gate/up tiles): a_scale[row_token[r]] scales row r's gate and
-// up values before the SiLU (the per-token RMSNorm scale of x: the norm weight is
-// folded into the packed w1 / w2 rows, and a per-row scale commutes with the product).
-template <bool GATE_UP, bool FP8, bool GATHER, bool SAVE_GU, bool RSCALE>
+// a_scale per A row, b_scale per B row (global row index).
+template <bool GATE_UP, bool SAVE_GU>
 __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds, const SlotTable& st, int E,
-                                                int n_tiles, int base, int n_full) {
-  constexpr bool M16 = !FP8;
-  constexpr int MA = M16 ? 8 : 4;    // A blocks of a wave
-  constexpr int NBB = M16 ? 8 : 4;   // B blocks of a wave
-  using Acc = std::conditional_t<M16, f32x4_t, f32x16_t>;
-  constexpr int ACCN = M16 ? 4 : 16;
-  constexpr int NSUB = KB / 64;               // MFMA K-substeps per step (bf16: 32 of K, fp8: 64)
+                                                int n_tiles, int n_cu, int base, int n_full) {
+  constexpr int MA = 4, NBB = 4;              // 32-row A and B blocks of a wave
+  constexpr int NSUB = KB / 64;               // MFMA K-substeps per step (64 of K)
   constexpr int NBLK = 2 * BLK_PER_WAVE;      // load blocks per wave per step: A, then B
-  static_assert(!RSCALE || (GATE_UP && GATHER && !FP8 && !SAVE_GU), "row scales are for bf16 gathered gate/up tiles");
   static_assert(!SAVE_GU || GATE_UP, "g/u saving is for gate/up tiles");
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 31, lh = lane >> 5;
-  const int r16 = lane & 15, lq = lane >> 4;
   const int wm = wave >> 1, wn = wave & 1;
   const int nk = g.k_bytes / KB;
   int L = blockIdx.x;
@@ -879,7 +900,6 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
 
   // slot table to LDS (every wave holds the same: wave 0 writes it; read after a barrier)
   int* const slot_l = reinterpret_cast<int*>(lds + FT_SLOTS);
-  int* const tok_l = reinterpret_cast<int*>(lds + FT_TOK);
   float* const sc_l = reinterpret_cast<float*>(lds + FT_SCALE);
   {
     int incl = st.ns;
@@ -924,12 +944,7 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
   // block covers bytes [16l, 16l+16) of it (tile row 8q + l/8, physical chunk l%8) and so
   // loads the logical chunk that swz() maps there: the LDS write of a block is one
   // contiguous, conflict-free 1 KiB.
-  // Tile rows past the expert's end load zeros instead: an offset beyond the buffer
-  // window's 2 GiB record count makes the hardware return 0 without a memory access
-  // (the scalar K offset is not range-checked, the per-lane offset is).  Their results
-  // are never stored; zero operands spare the memory traffic and the MFMA power of
-  // real data (the expert GEMMs run power-limited).
-  constexpr uint32_t OOB = 0x80000000u;
+  constexpr uint32_t OOB = 0x80000000u;  // an offset past every buffer window
   const int rsub = lane / CPR, pc = lane % CPR;
   uint32_t a_off[BLK_PER_WAVE], b_off[BLK_PER_WAVE];
 #pragma unroll
@@ -941,42 +956,26 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
   }
   __amdgpu_buffer_rsrc_t arsrc, brsrc;
   int koff = 0;
-  // points the loads at tile t.  GATHER: its rows' tokens are in tok_l; else the offsets are
-  // the same for every tile and the window ends at the expert's last row
-  auto aim = [&](const Tile& t) {
+  // points the loads at tile t (any = false: at nothing).  The A window ends at the
+  // expert's last row; loads past a window return zeros without a memory access (the
+  // scalar K offset is not range-checked, the per-lane offset is): the rows past the end
+  // are never stored, and zero operands spare traffic and MFMA power.
+  auto aim = [&](const Tile& t, bool any) {
     const int rows = t.m_end - t.m0;
-    brsrc = make_rsrc(g.B + ((int64_t)t.e * g.b_expert_rows + (int64_t)t.nt * BN) * g.ldb_bytes);
-    if constexpr (GATHER) {
-      arsrc = make_rsrc(g.A);
-      const int fl = fresh(lane), rsub = fl / CPR, pc = fl % CPR;
-#pragma unroll
-      for (int q = 0; q < BLK_PER_WAVE; ++q) {
-        const int tr = (wave * BLK_PER_WAVE + q) * RPB + rsub;
-        const uint32_t chunk = (uint32_t)(pc ^ ((tr >> 1) & (CPR - 1))) << 4;
-        const uint32_t off = (uint32_t)tok_l[tr] * (uint32_t)g.lda_bytes + chunk;
-        a_off[q] = tr < rows ? off : OOB + chunk;
-      }
-    } else {
-      arsrc = make_rsrc_window(g.A + (int64_t)t.m0 * g.lda_bytes, (int64_t)rows * g.lda_bytes);
-    }
+    brsrc = make_rsrc_window(g.B + ((int64_t)t.e * g.b_expert_rows + (int64_t)t.nt * BN) * g.ldb_bytes,
+                             any ? 0x7fffffff : 0);
+    arsrc = make_rsrc_window(g.A + (int64_t)t.m0 * g.lda_bytes, any ? (int64_t)rows * g.lda_bytes : 0);
   };
-  // thread tid looks up tile row tid: its activation row (GATHER) and its scales
-  auto look_token = [&](const Tile& t) -> int {
-    const int r = t.m0 + fresh(tid);
-    return r < t.m_end ? g.row_token[r] : 0;
-  };
-  auto look_scales = [&](const Tile& t, int tok, float& sa, float& sb) {
+  // thread tid looks up the scales of tile row tid and of B row tid
+  auto look_scales = [&](const Tile& t, float& sa, float& sb) {
     const int ft = fresh(tid), r = t.m0 + ft;
-    if constexpr (FP8) {
-      sa = r < t.m_end ? g.a_scale[r] : 0.0f;
-      sb = g.b_scale[(int64_t)t.e * g.b_expert_rows + (int64_t)t.nt * BN + ft];
-    }
-    if constexpr (RSCALE) sa = r < t.m_end ? g.a_scale[tok] : 0.0f;
+    sa = r < t.m_end ? g.a_scale[r] : 0.0f;
+    sb = g.b_scale[(int64_t)t.e * g.b_expert_rows + (int64_t)t.nt * BN + ft];
   };
   auto put_scales = [&](int set, float sa, float sb) {
     const int ft = fresh(tid);
-    if constexpr (FP8 || RSCALE) sc_l[set * 2 * BM + ft] = sa;
-    if constexpr (FP8) sc_l[set * 2 * BM + BM + ft] = sb;
+    sc_l[set * 2 * BM + ft] = sa;
+    sc_l[set * 2 * BM + BM + ft] = sb;
   };
 
   i32x4_t stg[NBLK];  // one step of this wave's tile data
@@ -994,25 +993,16 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
     *reinterpret_cast<i32x4_t*>(dst + lane * 16) = stg[qq];
   };
 
-  Acc acc[MA][NBB];
-  Frag<FP8> fa[2][MA], fb[2][NBB];
-  auto rdB = [&](int s, int i, int j, Frag<FP8>& b) {
-    if constexpr (M16)
-      read_frag16(lb_buf(s), b_lds_row<GATE_UP, 4>(wn, j >> 1, 16 * (j & 1) + r16), i, lq, b);
-    else
-      read_frag<FP8>(lb_buf(s), b_lds_row<GATE_UP, 4>(wn, j, lr), i, lh, b);
-  };
-  auto rdA = [&](int s, int i, int mi, Frag<FP8>& a) {
-    if constexpr (M16)
-      read_frag16(la_buf(s), wm * 128 + mi * 16 + r16, i, lq, a);
-    else
-      read_frag<FP8>(la_buf(s), wm * 128 + mi * 32 + lr, i, lh, a);
-  };
-  auto mma1 = [&](Acc& c, const Frag<FP8>& b, const Frag<FP8>& a) {
-    if constexpr (M16)
-      mfma16(c, b, a);
-    else
-      mfma<FP8>(c, b, a);
+  f32x16_t acc[MA][NBB];
+  Frag<true> fa[2][MA], fb[2][NBB];
+  auto rd = [&](int s, int i, auto nma_tag, Frag<true> (&a)[MA], Frag<true> (&b)[NBB]) {
+    constexpr int NMA = decltype(nma_tag)::value;
+    if constexpr (NMA > 0) {
+#pragma unroll
+      for (int mi = 0; mi < NMA; ++mi) read_frag<true>(la_buf(s), wm * 128 + mi * 32 + lr, i, lh, a[mi]);
+#pragma unroll
+      for (int j = 0; j < NBB; ++j) read_frag<true>(lb_buf(s), b_lds_row<GATE_UP, 4>(wn, j, lr), i, lh, b[j]);
+    }
   };
 
   // One K-step on stage cur while the registers hold the following step's data: those
@@ -1022,123 +1012,19 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
   // last substep the wave waits for its LDS writes and reads, then one barrier publishes
   // stage cur ^ 1, whose first fragments are read under the remaining MFMAs.  Register
   // dependencies give the vmcnt waits.
-  // bf16 (16x16 blocks): emitted in program order, one MFMA at a time, each followed by
-  // the LDS reads, block writes or reloads assigned to it and fenced with sched_barrier.
-  // (With scheduling groups the scheduler may take the MFMAs out of order, and the
-  // register allocator then stops tying each MFMA's accumulator input to its output:
-  // hundreds of accumulator copies per K-step.)  A 16x16x32 MFMA keeps the matrix pipe 16
-  // cycles, about what a 1 KiB LDS block write takes to issue, so the schedule gives each
-  // MFMA at most one LDS or memory instruction where it can.  Substep i uses B fragment set
-  // fb[i] and the one A set fa[0]; MFMAs go row block by row block.  Substep 0 reads
-  // substep 1's B fragments into fb[1] and each row block's next A fragment right after
-  // that row block's last MFMA (an A ring: no second A set).  Substep 1 meets the other
-  // waves at the barrier after MFMA GB, then reads the next stage's substep-0 fragments
-  // (B0, A0, B1, ..., each A after its row block's last MFMA).
-  auto step16 = [&](int cur, auto nab_tag) {
-    constexpr int NAB = decltype(nab_tag)::value;
-    constexpr int NMS = NAB * NBB;  // MFMAs per substep
-    constexpr bool FULL = NMS == 64;
-    constexpr int NR = NMS > 0 ? ((NBB + NAB) < NMS - 1 ? NBB + NAB : NMS - 1) : 0;
-    constexpr int GB = FULL ? 31 : NMS - 1 - NR;
-    constexpr int H0 = NBLK / 2;  // block writes in substep 0 (the rest in substep 1)
-    const int nxt = cur ^ 1;
-    static_for<0, 2>([&](auto ic) {
-      constexpr int i = decltype(ic)::value;
-      constexpr int NW = i == 0 ? H0 : NBLK - H0, QB = i == 0 ? 0 : H0;
-      if constexpr (NMS == 0) {
-        // a wave without rows: only its share of the tile loads and the barrier
-        static_for<0, NW>([&](auto wc) {
-          write_block(QB + decltype(wc)::value, nxt);
-          load_block(QB + decltype(wc)::value);
-        });
-        if constexpr (i == 1) {
-          wait_lgkmcnt0();
-          barrier_nofence();
-        }
-      } else {
-        // MFMA after which block write w / its reload go
-        constexpr auto w_at = [](int w) constexpr {
-          if (FULL) return i == 0 ? 16 + 6 * w : 4 * w;
-          const int span = i == 0 ? NMS - 2 : GB - 2;
-          return span > 0 ? 1 + (w * span) / NW : 0;
-        };
-        constexpr auto l_at = [](int w) constexpr {
-          if (FULL) return i == 0 ? 18 + 6 * w : 4 * w + 2;
-          const int span = i == 0 ? NMS - 2 : GB - 2;
-          return span > 0 ? 1 + (w * span) / NW : 0;
-        };
-        // substep 0: MFMA after which next-substep read B_j goes
-        constexpr auto b0_at = [](int j) constexpr { return FULL ? 2 * j : (j < NMS ? j : NMS - 1); };
-        // substep 1: post-barrier read k (0: B0, 1: A0, 2 ..: B1 .. B_{NBB-1}, then A1 ..)
-        constexpr auto post_at = [](int k, int kind, int idx) constexpr {
-          const int e0 = GB + 1 + (FULL ? 2 * k + 1 : k);
-          const int e1 = kind == 1 ? idx * NBB + NBB - 1 : 0;
-          const int at = e0 > e1 ? e0 : e1;
-          return at < NMS - 1 ? at : NMS - 1;
-        };
-        static_for<0, NMS>([&](auto gc) {
-          constexpr int gi = decltype(gc)::value;
-          constexpr int mi = gi / NBB, j = gi % NBB;
-          mma1(acc[mi][j], fb[i][j], fa[0][mi]);
-          __builtin_amdgcn_sched_barrier(0);
-          // block writes, then reloads (substep 1: all before the barrier)
-          static_for<0, NW>([&](auto wc) {
-            constexpr int w = decltype(wc)::value;
-            if constexpr (w_at(w) == gi) write_block(QB + w, nxt);
-          });
-          static_for<0, NW>([&](auto wc) {
-            constexpr int w = decltype(wc)::value;
-            if constexpr (l_at(w) == gi) load_block(QB + w);
-          });
-          if constexpr (i == 0) {
-            static_for<0, NBB>([&](auto jc) {
-              constexpr int jj = decltype(jc)::value;
-              if constexpr (b0_at(jj) == gi) rdB(cur, 1, jj, fb[1][jj]);
-            });
-            if constexpr (j == NBB - 1) rdA(cur, 1, mi, fa[0][mi]);
-          } else {
-            if constexpr (gi == GB) {
-              wait_lgkmcnt0();
-              barrier_nofence();
-            }
-            static_for<0, NBB + NAB>([&](auto kc) {
-              constexpr int k = decltype(kc)::value;
-              constexpr int kind = k == 0 ? 0 : k == 1 ? 1 : k < NBB + 1 ? 0 : 1;
-              constexpr int idx = k == 0 ? 0 : k == 1 ? 0 : k < NBB + 1 ? k - 1 : k - NBB;
-              if constexpr (post_at(k, kind, idx) == gi) {
-                if constexpr (kind == 0)
-                  rdB(nxt, 0, idx, fb[0][idx]);
-                else
-                  rdA(nxt, 0, idx, fa[0][idx]);
-              }
-            });
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        });
-      }
-    });
-  };
-  // fp8 (32x32 blocks): half of the block writes and reloads in each of the two substeps,
+  // Half of the block writes and reloads go in each of the two substeps,
   // fragments double buffered, interleaved by scheduling groups; in the last substep the
   // writes and most MFMAs go out before the wait and the barrier (the MFMAs read registers
   // only), so the MFMA pipe is busy while the waves meet.
-  auto step32 = [&](int cur, auto nma_tag) {
+  auto step = [&](int cur, auto nma_tag) {
     constexpr int NMA = decltype(nma_tag)::value;
     constexpr int RD = NMA > 0 ? 2 * (NMA + NBB) : 0;  // LDS reads of a substep's fragments
     constexpr int NMS = NMA * NBB;
     const int nxt = cur ^ 1;
-    auto rd = [&](int s, int i, Frag<FP8> (&a)[MA], Frag<FP8> (&b)[NBB]) {
-      if constexpr (NMA > 0) {
-#pragma unroll
-        for (int mi = 0; mi < NMA; ++mi) rdA(s, i, mi, a[mi]);
-#pragma unroll
-        for (int j = 0; j < NBB; ++j) rdB(s, i, j, b[j]);
-      }
-    };
-    auto mma_part = [&](const Frag<FP8> (&a)[MA], const Frag<FP8> (&b)[NBB], auto lo_tag, auto hi_tag) {
+    auto mma_part = [&](const Frag<true> (&a)[MA], const Frag<true> (&b)[NBB], auto lo_tag, auto hi_tag) {
       static_for<decltype(lo_tag)::value, decltype(hi_tag)::value>([&](auto xc) {
         constexpr int x = decltype(xc)::value;
-        mma1(acc[x / NBB][x % NBB], b[x % NBB], a[x / NBB]);
+        mfma<true>(acc[x / NBB][x % NBB], b[x % NBB], a[x / NBB]);
       });
     };
     static_for<0, NSUB>([&](auto ic) {
@@ -1146,7 +1032,7 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
       constexpr int bi = i & 1;
       constexpr int q0 = i * NBLK / NSUB, q1 = (i + 1) * NBLK / NSUB;
       constexpr int nq = q1 - q0;
-      if constexpr (i + 1 < NSUB) rd(cur, i + 1, fa[bi ^ 1], fb[bi ^ 1]);
+      if constexpr (i + 1 < NSUB) rd(cur, i + 1, nma_tag, fa[bi ^ 1], fb[bi ^ 1]);
       static_for<q0, q1>([&](auto qc) { write_block(decltype(qc)::value, nxt); });
       static_for<q0, q1>([&](auto qc) { load_block(decltype(qc)::value); });
       if constexpr (i + 1 < NSUB) {
@@ -1162,7 +1048,7 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
         __builtin_amdgcn_sched_barrier(0);
         wait_lgkmcnt0();
         barrier_nofence();
-        rd(nxt, 0, fa[bi ^ 1], fb[bi ^ 1]);
+        rd(nxt, 0, nma_tag, fa[bi ^ 1], fb[bi ^ 1]);
         if constexpr (NA > 0) {
           mma_part(fa[bi], fb[bi], std::integral_constant<int, NMS - NA>{}, std::integral_constant<int, NMS>{});
           sched_spread<NA, RD, 0, 0>();
@@ -1178,7 +1064,7 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
   auto epilogue = [&](const Tile& t, int set, auto nma_tag) {
     constexpr int NMA = decltype(nma_tag)::value;
     if constexpr (NMA > 0) {
-      const int fl = fresh(lane), r16 = fl & 15, lq = fl >> 4, lr = fl & 31, lh = fl >> 5;
+      const int fl = fresh(lane), lr = fl & 31, lh = fl >> 5;
       const float* const sa_l = sc_l + set * 2 * BM;
       const float* const sb_l = sa_l + BM;
       const __amdgpu_buffer_rsrc_t crsrc = make_rsrc(g.C + (int64_t)t.m0 * g.ldc);
@@ -1186,106 +1072,52 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
       const int rows = t.m_end - t.m0;
       const uint32_t ldc2 = (uint32_t)g.ldc * 2u;
       const int col0 = (GATE_UP ? t.nt * 128 : t.nt * 256) + wn * (GATE_UP ? 64 : 128);
-      if constexpr (M16) {
-        constexpr int NJ = GATE_UP ? NBB / 2 : NBB;
-        // the lane's piece: row r16 % 8 (+ 8 in the second store), 16-byte column chunk of
-        // the 64-column (128-byte) group
-        const bool low = r16 < 8;
-        const int lcol = (low ? 0 : 32) + (lq & 1) * 16 + (lq >> 1) * 8;
-        // the row segments of blocks b .. b + 3 (64 columns from column `col`)
-        auto put = [&](__amdgpu_buffer_rsrc_t rs, int mi, uint32_t stride2, int col, int valid, auto&& four) {
-          i32x4_t p = merge16(four(0), four(1)), q = merge16(four(2), four(3));
-          swap_halves(p, q, low);
-          const int row = wm * 128 + mi * 16 + (r16 & 7);
-          const uint32_t off = (uint32_t)row * stride2 + 2u * (uint32_t)(col + lcol);
-          const bool in = col + lcol < valid;
-          __builtin_amdgcn_raw_buffer_store_b128(p, rs, in && row < rows ? off : OOB, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b128(q, rs, in && row + 8 < rows ? off + 8u * stride2 : OOB, 0, 0);
-        };
+      constexpr int NJ = GATE_UP ? NBB / 2 : NBB;
 #pragma unroll
-        for (int mi = 0; mi < 2 * NMA; ++mi) {
-          const float sar = RSCALE ? sa_l[wm * 128 + mi * 16 + r16] : 1.0f;
+      for (int mi = 0; mi < NMA; ++mi) {
+        const int row = wm * 128 + mi * 32 + lr;
+        const float sar = sa_l[row];
+        const uint32_t roff = row < rows ? (uint32_t)row * ldc2 : OOB;
+        const uint32_t goff = row < rows ? (uint32_t)row * 2u * ldc2 : OOB;
 #pragma unroll
-          for (int jp = 0; jp < NJ; jp += 4) {
-            put(crsrc, mi, ldc2, col0 + jp * 16, g.n_valid, [&](int h) {
-              float f[4];
+        for (int jo = 0; jo < NJ; ++jo) {
 #pragma unroll
-              for (int c = 0; c < 4; ++c) {
+          for (int cp = 0; cp < 4; cp += 2) {
+            i32x2_t v[2], vg[2], vu[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const int c = cp + h;
+              const f32x4_t sb =
+                  *reinterpret_cast<const f32x4_t*>(sb_l + b_lds_row<GATE_UP, 4>(wn, jo, 8 * c + 4 * lh));
+              float f[4], gv[4], uv[4];
+              f32x4_t su = sb;
+              if constexpr (GATE_UP)
+                su = *reinterpret_cast<const f32x4_t*>(sb_l + b_lds_row<GATE_UP, 4>(wn, jo + NBB / 2, 8 * c + 4 * lh));
+#pragma unroll
+              for (int q = 0; q < 4; ++q) {
+                gv[q] = acc[mi][jo][4 * c + q] * (sar * sb[q]);
                 if constexpr (GATE_UP) {
-                  float gg = acc[mi][jp + h][c], u = acc[mi][jp + h + NBB / 2][c];
-                  if constexpr (RSCALE) {
-                    gg *= sar;
-                    u *= sar;
-                  }
-                  f[c] = silu_fast_f32(gg) * u;
+                  uv[q] = acc[mi][jo + NBB / 2][4 * c + q] * (sar * su[q]);
+                  f[q] = silu_fast_f32(gv[q]) * uv[q];
                 } else {
-                  f[c] = acc[mi][jp + h][c];
+                  f[q] = gv[q];
                 }
               }
-              return pack4_bf16(f[0], f[1], f[2], f[3]);
-            });
-          }
-          __builtin_amdgcn_sched_barrier(0);  // one row block's temporaries at a time
-          if constexpr (SAVE_GU) {
-            // the pre-activation values in the packed column order, row stride 2 ldc: per
-            // 128 columns of h, 128 gate then 128 up columns
-#pragma unroll
-            for (int j = 0; j < NBB; j += 4) {
-              put(grsrc, mi, 2u * ldc2, t.nt * 256 + b_lds_row<true, 4>(wn, j >> 1, 0), 1 << 30, [&](int h) {
-                return pack4_bf16(acc[mi][j + h][0], acc[mi][j + h][1], acc[mi][j + h][2], acc[mi][j + h][3]);
-              });
-            }
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        }
-      } else {
-        constexpr int NJ = GATE_UP ? NBB / 2 : NBB;
-#pragma unroll
-        for (int mi = 0; mi < NMA; ++mi) {
-          const int row = wm * 128 + mi * 32 + lr;
-          const float sar = sa_l[row];
-          const uint32_t roff = row < rows ? (uint32_t)row * ldc2 : OOB;
-          const uint32_t goff = row < rows ? (uint32_t)row * 2u * ldc2 : OOB;
-#pragma unroll
-          for (int jo = 0; jo < NJ; ++jo) {
-#pragma unroll
-            for (int cp = 0; cp < 4; cp += 2) {
-              i32x2_t v[2], vg[2], vu[2];
-#pragma unroll
-              for (int h = 0; h < 2; ++h) {
-                const int c = cp + h;
-                const f32x4_t sb =
-                    *reinterpret_cast<const f32x4_t*>(sb_l + b_lds_row<GATE_UP, 4>(wn, jo, 8 * c + 4 * lh));
-                float f[4], gv[4], uv[4];
-                f32x4_t su = sb;
-                if constexpr (GATE_UP)
-                  su = *reinterpret_cast<const f32x4_t*>(sb_l + b_lds_row<GATE_UP, 4>(wn, jo + NBB / 2, 8 * c + 4 * lh));
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                  gv[q] = acc[mi][jo][4 * c + q] * (sar * sb[q]);
-                  if constexpr (GATE_UP) {
-                    uv[q] = acc[mi][jo + NBB / 2][4 * c + q] * (sar * su[q]);
-                    f[q] = silu_fast_f32(gv[q]) * uv[q];
-                  } else {
-                    f[q] = gv[q];
-                  }
-                }
-                v[h] = pack4_bf16(f[0], f[1], f[2], f[3]);
-                if constexpr (SAVE_GU) {
-                  vg[h] = pack4_bf16(gv[0], gv[1], gv[2], gv[3]);
-                  vu[h] = pack4_bf16(uv[0], uv[1], uv[2], uv[3]);
-                }
-              }
-              const int lcol = 8 * (cp + lh);
-              const int col = col0 + jo * 32 + lcol;
-              const uint32_t off = col < g.n_valid ? roff + 2u * (uint32_t)col : OOB;
-              __builtin_amdgcn_raw_buffer_store_b128(merge32(v[0], v[1]), crsrc, off, 0, 0);
+              v[h] = pack4_bf16(f[0], f[1], f[2], f[3]);
               if constexpr (SAVE_GU) {
-                const uint32_t cg = (uint32_t)(t.nt * 256 + b_lds_row<true, 4>(wn, jo, 0) + lcol);
-                const uint32_t cu = (uint32_t)(t.nt * 256 + b_lds_row<true, 4>(wn, jo + NBB / 2, 0) + lcol);
-                __builtin_amdgcn_raw_buffer_store_b128(merge32(vg[0], vg[1]), grsrc, goff + 2u * cg, 0, 0);
-                __builtin_amdgcn_raw_buffer_store_b128(merge32(vu[0], vu[1]), grsrc, goff + 2u * cu, 0, 0);
+                vg[h] = pack4_bf16(gv[0], gv[1], gv[2], gv[3]);
+                vu[h] = pack4_bf16(uv[0], uv[1], uv[2], uv[3]);
               }
+            }
+            const int lcol = 8 * (cp + lh);
+            const int col = col0 + jo * 32 + lcol;
+            const uint32_t off = col < g.n_valid ? roff + 2u * (uint32_t)col : OOB;
+            __builtin_amdgcn_raw_buffer_store_b128(merge32(v[0], v[1]), crsrc, off, 0, 0);
+            if constexpr (SAVE_GU) {
+              const uint32_t cg = (uint32_t)(t.nt * 256 + b_lds_row<true, 4>(wn, jo, 0) + lcol);
+              const uint32_t cu = (uint32_t)(t.nt * 256 + b_lds_row<true, 4>(wn, jo + NBB / 2, 0) + lcol);
+              __builtin_amdgcn_raw_buffer_store_b128(merge32(vg[0], vg[1]), grsrc, goff + 2u * cg, 0, 0);
+              __builtin_amdgcn_raw_buffer_store_b128(merge32(vu[0], vu[1]), grsrc, goff + 2u * cu, 0, 0);
             }
           }
         }
@@ -1297,17 +1129,10 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
   // in registers)
   Tile cur = decode(L);
   {
-    int tok = 0;
-    if constexpr (GATHER) tok = look_token(cur);
-    float sa = 0.0f, sb = 0.0f;
-    if constexpr (FP8 || RSCALE) look_scales(cur, tok, sa, sb);
-    if constexpr (GATHER) {
-      if (g.row_index) tok = g.row_index[tok];
-      tok_l[tid] = tok;
-      __syncthreads();
-    }
+    float sa, sb;
+    look_scales(cur, sa, sb);
     put_scales(0, sa, sb);
-    aim(cur);
+    aim(cur, true);
     koff = 0;
 #pragma unroll
     for (int qq = 0; qq < NBLK; ++qq) load_block(qq);
@@ -1323,35 +1148,22 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
   int set = 0;  // scale set of the tile
   bool more;
   do {
-    more = L + (int)gridDim.x < n_full;
-    if (more) L += (int)gridDim.x;
-    const Tile nx = decode(L);  // the last tile's last loads are its own first steps again
+    more = L + n_cu < n_full;
+    if (more) L += n_cu;
+    const Tile nx = decode(L);
     auto body = [&](auto nma_tag) {
       constexpr int NMA = decltype(nma_tag)::value;
-      constexpr auto blk = std::integral_constant<int, M16 ? 2 * NMA : NMA>{};
-      constexpr int NAB = decltype(blk)::value;
       if constexpr (NMA > 0) {
+        rd(par, 0, nma_tag, fa[0], fb[0]);
 #pragma unroll
-        for (int j = 0; j < NBB; ++j) rdB(par, 0, j, fb[0][j]);
-#pragma unroll
-        for (int mi = 0; mi < NAB; ++mi) rdA(par, 0, mi, fa[0][mi]);
-#pragma unroll
-        for (int i = 0; i < NAB; ++i)
+        for (int i = 0; i < NMA; ++i)
 #pragma unroll
           for (int j = 0; j < NBB; ++j)
 #pragma unroll
-            for (int r = 0; r < ACCN; ++r) acc[i][j][r] = 0.0f;
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
       }
-      int tok = 0;
-      float sa = 0.0f, sb = 0.0f;
-      if constexpr (GATHER) tok = look_token(nx);
-      if constexpr (FP8) look_scales(nx, 0, sa, sb);
-      auto step = [&](int s) {
-        if constexpr (M16)
-          step16(s, blk);
-        else
-          step32(s, blk);
-      };
+      float sa, sb;
+      look_scales(nx, sa, sb);
 #pragma unroll 1
       for (int kt = 0; kt < nk; ++kt) {
         koff = (kt + 2) * KB;
@@ -1359,30 +1171,22 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
           // the last two steps load the next tile's first two
           koff = (kt + 2 - nk) * KB;
           if (kt == nk - 2) {
-            if constexpr (RSCALE) look_scales(nx, tok, sa, sb);
             // (with two steps nothing else keeps this write behind the other waves' reads of
             // the set in the previous tile's epilogue)
-            if ((FP8 || RSCALE) && nk == 2) barrier_nofence();
+            if (nk == 2) barrier_nofence();
             put_scales(set ^ 1, sa, sb);
-            if constexpr (GATHER) {
-              if (g.row_index) tok = g.row_index[tok];
-              tok_l[fresh(tid)] = tok;
-              wait_lgkmcnt0();
-              barrier_nofence();
-            }
-            aim(nx);
+            aim(nx, more);
           }
         }
-        step((par + kt) & 1);
+        step((par + kt) & 1, nma_tag);
       }
-      // every accumulator leaves the loop in AGPRs (without this the allocator takes some of
-      // them through VGPRs in the loop, with copies around their MFMAs)
-      if constexpr (M16) {
+      // every accumulator leaves the loop in AGPRs, and the epilogue stays out of its last
+      // step (else the allocator spills in the loop)
 #pragma unroll
-        for (int i = 0; i < NAB; ++i)
+      for (int i = 0; i < NMA; ++i)
 #pragma unroll
-          for (int j = 0; j < NBB; ++j) asm volatile("" : "+a"(acc[i][j]));
-      }
+        for (int j = 0; j < NBB; ++j) asm volatile("" : "+a"(acc[i][j]));
+      __builtin_amdgcn_sched_barrier(0);
       epilogue(cur, set, nma_tag);
     };
     // row blocks of this wave holding rows (wave-uniform): 4 (more than 64 rows), 2, 0
@@ -1399,14 +1203,17 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
   } while (more);
 }
 
-// Work of workgroup blockIdx.x of a grid of at most one workgroup per CU (n_cu).  The
-// tiles (slot, column tile) are numbered densely (dense_tile); the first R = N / n_cu full
-// rounds of tiles go to gemm_full_tiles in the XCD-aware order.  The N - R n_cu tiles left
-// would occupy few compute units for a whole tile time, so when they fit (split > 1: at
-// most n_cu / split of them) each is split into `split` narrow tiles of 1/split of its
-// columns (the full K), which all run at once, one per workgroup.  A narrow tile
-// computes every output element with the same MFMA sequence as the full tile, so the
-// results are identical.  split = 1 keeps the tail tiles whole.
+// Work of workgroup blockIdx.x.  The tiles (slot, column tile) are numbered densely
+// (dense_tile); with n_cu workgroups resident at a time, the first R = N/n_cu full
+// rounds take one tile per workgroup in the XCD-aware order.  The N - R n_cu tiles
+// left would occupy few compute units for a whole tile time, so when they fit
+// (split > 1: at most n_cu / split of them) each is split into `split` narrow tiles
+// of 1/split of its columns (the full K), which all run at once.  A narrow tile
+// computes every output element with the same MFMA sequence as the full tile, so
+// the results are identical.  split = 1 keeps the tail tiles whole.
+// e4m3 products of at least two K-steps: the full rounds (and whole tail tiles) go to
+// gemm_full_tiles on the first n_cu workgroups, the narrow tiles to the ones after them (a
+// single K-step: all tiles in halves).
 template <bool GATE_UP, bool FP8, bool GATHER, bool SAVE_GU = false, bool RSCALE = false>
 __global__ __launch_bounds__(GEMM_THREADS, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void grouped_gemm_kernel(
     GemmArgs g, const int32_t* __restrict__ offsets, int E, int n_tiles, int n_cu) {
@@ -1414,25 +1221,64 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) __attribute__((amdgpu_waves_per_eu
   __shared__ __attribute__((aligned(1024))) uint8_t lds[GEMM_LDS];
   const SlotTable st = load_slots(offsets, E);
   const int n_all = st.n_slots * n_tiles;
-  const int base = n_all / n_cu * n_cu, n_rest = n_all - base;
-  int split = n_rest == 0 ? 1 : 4 * n_rest <= n_cu ? 4 : 2 * n_rest <= n_cu ? 2 : 1;
-  int n_full = split == 1 ? n_all : base;
-  if (g.k_bytes < 2 * KB) {
-    // a single K-step: all tiles in halves
-    n_full = 0;
-    split = 2;
+  const int rounds = n_all / n_cu, base = rounds * n_cu, n_rest = n_all - base;
+  int split = 1;
+  if (n_rest > 0) {
+    if (4 * n_rest <= n_cu)
+      split = 4;
+    else if (2 * n_rest <= n_cu)
+      split = 2;
   }
-  gemm_full_tiles<GATE_UP, FP8, GATHER, SAVE_GU, RSCALE>(g, lds, st, E, n_tiles, base, n_full);
-  for (int u = blockIdx.x; u < (n_all - n_full) * split; u += gridDim.x) {
-    const int t = n_full + u / split, q = u % split;
+  const int L = blockIdx.x;
+  if constexpr (FP8) {
+    const bool one_step = g.k_bytes < 2 * KB;
+    if (one_step)
+      split = 2;
+    else if (L < n_cu) {
+      gemm_full_tiles<GATE_UP, SAVE_GU>(g, lds, st, E, n_tiles, n_cu, base, split == 1 ? n_all : base);
+      return;
+    }
+    const int first = one_step ? 0 : base, u = one_step ? L : L - n_cu;
+    if (split == 1 || u >= (n_all - first) * split) return;
+    int slot, nt, e, m0, m_end;
+    dense_tile(first + u / split, st.n_slots, n_tiles, slot, nt);
+    find_slot(st, E, slot, e, m0, m_end);
+    if (split == 2)
+      gemm_tile<GATE_UP, true, false, 2, SAVE_GU, false>(g, lds, e, m0, m_end, nt, u % split);
+    else
+      gemm_tile<GATE_UP, true, false, 1, SAVE_GU, false>(g, lds, e, m0, m_end, nt, u % split);
+    return;
+  } else {
+    int t, q = 0;
+    if (L < base) {
+      t = (base % (NXCD * SB_TILES)) == 0 ? xcd_tile(L) : L;
+    } else if (split == 1) {
+      if (L >= n_all) return;
+      t = L;
+    } else {
+      const int u = L - base;
+      if (u >= n_rest * split) return;
+      t = base + u / split;
+      q = u % split;
+    }
     int slot, nt, e, m0, m_end;
     dense_tile(t, st.n_slots, n_tiles, slot, nt);
     find_slot(st, E, slot, e, m0, m_end);
-    __syncthreads();  // the last tile's stages are reused
-    if (split == 2)
-      narrow_tile<GATE_UP, FP8, GATHER, 2, SAVE_GU, RSCALE>(g, lds, e, m0, m_end, nt, q);
+    if (L < base || split == 1) {
+      // row blocks of this wave holding rows (wave-uniform): 4 (more than 64 rows), 2, 1, 0
+      const int wrows = m_end - m0 - (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >> 1) * 128;
+      if (wrows > 64)
+        gemm_tile<GATE_UP, FP8, GATHER, 4, SAVE_GU, RSCALE, 4>(g, lds, e, m0, m_end, nt, 0);
+      else if (wrows > 32)
+        gemm_tile<GATE_UP, FP8, GATHER, 4, SAVE_GU, RSCALE, 2>(g, lds, e, m0, m_end, nt, 0);
+      else if (wrows > 0)
+        gemm_tile<GATE_UP, FP8, GATHER, 4, SAVE_GU, RSCALE, 1>(g, lds, e, m0, m_end, nt, 0);
+      else
+        gemm_tile<GATE_UP, FP8, GATHER, 4, SAVE_GU, RSCALE, 0>(g, lds, e, m0, m_end, nt, 0);
+    } else if (split == 2)
+      gemm_tile<GATE_UP, FP8, GATHER, 2, SAVE_GU, RSCALE>(g, lds, e, m0, m_end, nt, q);
     else
-      narrow_tile<GATE_UP, FP8, GATHER, 1, SAVE_GU, RSCALE>(g, lds, e, m0, m_end, nt, q);
+      gemm_tile<GATE_UP, FP8, GATHER, 1, SAVE_GU, RSCALE>(g, lds, e, m0, m_end, nt, q);
   }
 }
 
@@ -1454,5 +1300,4 @@ void launch_gate_up_rows(const GemmLaunch& l);                    // bf16, gathe
 void launch_gate_up_rows_gu(const GemmLaunch& l);                 // the same, saving the gate / up values
 void launch_permuted(const GemmLaunch& l, bool gate_up);          // bf16, permuted rows
 void launch_fp8(const GemmLaunch& l, bool gate_up, bool save_gu); // e4m3, permuted rows
-
 }  // namespace kmoe_tiles
