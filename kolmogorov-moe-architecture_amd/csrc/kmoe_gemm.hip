@@ -6,6 +6,30 @@ using namespace kmoe_tiles;
 
 namespace {
 
+// Slots of SMALL_ROWS rows that max_rows rows over E experts can fill: at most one per row,
+// and the full ones plus a partial one per expert.
+int64_t small_slots(int E, int64_t max_rows) { return std::min<int64_t>(max_rows, max_rows / SMALL_ROWS + E); }
+
+// Whether a bf16 product runs on the small-row kernel and not on the 256-row tiles.  Kernel
+// times in us of gate/up + down, small-row kernel / 256-row tiles:
+// - up to 10 rows per expert (max_rows / E), where a wave's weight rows are read once:
+//   d 2048, F 2816, 16 experts, top-2: 16 tokens 86 / 113, 48 tokens 106 / 122, 128 tokens
+//   (16 rows) 133 / 126;
+// - and wherever its grid is at most two workgroups per CU, as latency then counts: d 256,
+//   F 352, 4 experts: 128 tokens 10.0 / 15.9, 512 tokens 15.9 / 16.3 (down 6.3 / 8.2 at
+//   288 workgroups, gate/up 9.6 / 8.2 at 864).
+// (A kernel of 128-row slots for 10 to 64 rows per expert, weights to registers and rows
+// through LDS, measured 4% faster alone at 16 to 32 rows and 2% slower inside a layer.)
+bool small_rows_product(bool gate_up, int E, int64_t max_rows, int64_t b_expert_rows, int64_t ldb_bytes,
+                        int n_tiles) {
+  // lanes address an expert's weights with 31-bit offsets
+  if (b_expert_rows * ldb_bytes >= (int64_t)1 << 31) return false;
+  const int64_t cols = (int64_t)n_tiles * (gate_up ? BN / 2 : BN);
+  const int64_t wgs = small_slots(E, max_rows) * (cols / small_cols(gate_up));
+  if (wgs > 0x7fffffff) return false;
+  return max_rows <= 10 * (int64_t)E || wgs <= 2 * (int64_t)kmoe::cu_count();
+}
+
 // A rows: the permuted rows (row_token == nullptr) or gathered rows of the
 // activation matrix A (n_a_rows rows) through row_token / row_index.
 int launch_gemm(bool gate_up, bool fp8, const void* A, const float* a_scale, const int32_t* row_token,
@@ -53,7 +77,10 @@ int launch_gemm(bool gate_up, bool fp8, const void* A, const float* a_scale, con
     return KMOE_ERR_SHAPE;
   }
   const GemmLaunch l{g, offsets, E, n_tiles, n_cu, (unsigned)blocks, s};
-  if (fp8)
+  if (!fp8 && small_rows_product(gate_up, E, max_rows, b_expert_rows, g.ldb_bytes, n_tiles)) {
+    const int n_ct = n_tiles * (gate_up ? BN / 2 : BN) / small_cols(gate_up);
+    launch_small_rows(GemmLaunch{g, offsets, E, n_ct, n_cu, (unsigned)(small_slots(E, max_rows) * n_ct), s}, gate_up);
+  } else if (fp8)
     launch_fp8(l, gate_up, gu_out != nullptr);
   else if (row_token && gu_out)
     launch_gate_up_rows_gu(l);

@@ -1300,4 +1300,10 @@ void launch_gate_up_rows(const GemmLaunch& l);                    // bf16, gathe
 void launch_gate_up_rows_gu(const GemmLaunch& l);                 // the same, saving the gate / up values
 void launch_permuted(const GemmLaunch& l, bool gate_up);          // bf16, permuted rows
 void launch_fp8(const GemmLaunch& l, bool gate_up, bool save_gu); // e4m3, permuted rows
+// bf16, few rows per expert (kmoe_gemm_small.hip): slots of SMALL_ROWS rows, n_tiles column
+// tiles of small_cols() output columns
+constexpr int SMALL_ROWS = 32;
+inline int small_cols(bool gate_up) { return gate_up ? 16 : 32; }
+void launch_small_rows(const GemmLaunch& l, bool gate_up);
+
 }  // namespace kmoe_tiles

@@ -757,3 +757,52 @@ def test_full_tile_loop(dev, path, d):
         if gu is not None:
             packed = torch.cat([gg[:, :128], uu[:, :128], gg[:, 128:], uu[:, 128:]], 1)
             assert rel(gu[s:t], packed) <= 4e-3, (path, d, e, counts[e])
+
+
+# ------------------------------------------------------------------ few rows per expert
+@pytest.mark.parametrize("d,F,counts", [(64, 40, [1, 0, 2]), (128, 128, [16, 17, 1, 0]), (320, 130, [32, 33, 15, 31]),
+                                        (2048, 704, [1] + [0] * 6 + [3, 10, 64]), (192, 2816, [2, 1])])
+@pytest.mark.parametrize("path", ["rows", "row_index", "rscale", "save_gu", "permuted"])
+def test_small_rows(dev, path, d, F, counts):
+    """The small-row products (at most 10 rows per expert, or a small grid): K of one step
+    to more than the waves' ring, rows at the edges of the 16-row blocks and the 32-row
+    slots, experts without rows, F not a multiple of the packing; gate/up (gathered, through
+    a row index, row-scaled, g/u-saving, permuted) and down against fp32 matmuls of the
+    same operands (bar 4e-3 rel-L2: the bf16 rounding of each output is 2^-9 at most)."""
+    E, A = len(counts), sum(counts)
+    off_l = np.concatenate([[0], np.cumsum(counts)])
+    off = torch.tensor(off_l, dtype=torch.int32, device=dev)
+    g = torch.Generator(device=dev).manual_seed(d + F)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    T = 300
+    x = bf16(rnd(T, d))
+    w1, w2, w3 = (bf16(rnd(*s) * s[1] ** -0.5) for s in ((E, d, F), (E, d, F), (E, F, d)))
+    pw = ops.pack_weights(w1, w2, w3)
+    ri = torch.randperm(T, generator=g, device=dev).to(torch.int32)
+    rt = torch.randint(0, T, (A,), generator=g, device=dev, dtype=torch.int32)
+    rows = ri[rt.long()] if path == "row_index" else rt
+    rs = torch.rand(T, generator=g, device=dev) + 0.5
+    gu = None
+    if path == "permuted":
+        h = ops.gemm_gate_up(x[rt.long()].contiguous(), None, off, pw, A)
+    else:
+        h = ops.gemm_gate_up_rows(x, ri if path == "row_index" else None, rt, off, pw, A, save_gu=path == "save_gu",
+                                  rscale=rs if path == "rscale" else None)
+        if path == "save_gu":
+            h, gu = h
+    y = ops.gemm_down(h, None, off, pw, A)
+    xr = x[rows.long()].float() * (rs[rt.long(), None] if path == "rscale" else 1.0)
+    rel = lambda a, b: float((a.float() - b).norm() / b.norm())
+    for e in range(E):
+        s, t = int(off_l[e]), int(off_l[e + 1])
+        if s == t:
+            continue
+        gg, uu = xr[s:t] @ w1[e].float(), xr[s:t] @ w2[e].float()
+        assert rel(h[s:t, :F], torch.nn.functional.silu(gg) * uu) <= 4e-3, (e, counts[e])
+        assert not h[s:t, F:].any()
+        assert rel(y[s:t], h[s:t, :F].float() @ w3[e].float()) <= 4e-3, (e, counts[e])
+        if gu is not None:
+            for f in range(0, F, 128):
+                n = min(128, F - f)
+                assert rel(gu[s:t, 2 * f:2 * f + n], gg[:, f:f + n]) <= 4e-3
+                assert rel(gu[s:t, 2 * f + 128:2 * f + 128 + n], uu[:, f:f + n]) <= 4e-3
