@@ -488,6 +488,18 @@ int kmoe_router_rms(const void* x, const int32_t* row_index, int64_t T, int d, c
                     const void* w_out, int E, const float* logit_bias, int k, float* logits,
                     int64_t* topk_idx, float* topk_w, float* partials, float eps, float* rscale, void* stream);
 
+/* The token-choice bf16 layer forward as one call: kmoe_router_hist (with rms_eps >= 0:
+ * of RMSNorm(x), the norm weight folded into w_in and w13; rms_eps < 0: none),
+ * kmoe_dispatch_counted(_aux, with aux_out: 3 floats), the gathered gate/up and the down
+ * product and kmoe_combine_residual (residual may be NULL), T > 0 tokens, with the same
+ * results.  counts: E int32.  The workspace (kmoe_moe_forward_workspace_bytes, 256-byte
+ * aligned) holds every intermediate.                                          */
+size_t kmoe_moe_forward_workspace_bytes(int64_t T, int d, int E, int k, int F);
+int kmoe_moe_forward(const void* x, int64_t T, int d, const void* w_in, const void* w_out, int E,
+                     const float* logit_bias, int k, const void* w13_packed, const void* w3_packed, int F,
+                     int64_t capacity, float rms_eps, const void* residual, void* y, int y_dtype, int32_t* counts,
+                     float* aux_out, float w_lb, float w_z, void* workspace, size_t workspace_bytes, void* stream);
+
 /* kmoe_gemm_gate_up_rows on RMSNorm(x): the gate and up values of permuted row r are
  * scaled by rscale[row_token[r]] before the SiLU (w13 packed from the norm-folded
  * w1 / w2).  The normalised rows are never written.                           */

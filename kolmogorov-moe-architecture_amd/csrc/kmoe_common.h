@@ -31,6 +31,11 @@ int cu_count();
 // router's aux partials and block histograms, which the aux-loss and dispatch
 // reductions read.
 int router_block_tokens(int64_t T);
+// Every form of the router launch (kmoe_router.hip): rscale with RMSNorm folded in,
+// block_counts the per-block histograms, hidden_pre the training forward's.
+int router_launch(const void* x, const int32_t* row_index, int64_t T, int d, const void* w_in, const void* w_out,
+                  int E, const float* logit_bias, int k, float* logits, int64_t* topk_idx, float* topk_w,
+                  float* partials, float* hidden_pre, float eps, float* rscale, int32_t* block_counts, void* stream);
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 

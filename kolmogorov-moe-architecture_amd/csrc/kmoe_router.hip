@@ -400,7 +400,7 @@ extern "C" int64_t kmoe_router_partials_len(int64_t T, int E) {
   return kmoe::ceil_div<int64_t>(T, kmoe::router_block_tokens(T)) * (int64_t)(E + 1);
 }
 
-namespace {
+namespace kmoe {
 int router_launch(const void* x, const int32_t* row_index, int64_t T, int d, const void* w_in, const void* w_out,
                   int E, const float* logit_bias, int k, float* logits, int64_t* topk_idx, float* topk_w,
                   float* partials, float* hidden_pre, float eps, float* rscale, int32_t* block_counts,
@@ -463,7 +463,8 @@ int router_launch(const void* x, const int32_t* row_index, int64_t T, int d, con
 #undef KMOE_ROUTER_LAUNCH3
   return kmoe::check_launch("kmoe_router");
 }
-}  // namespace
+}  // namespace kmoe
+using kmoe::router_launch;
 
 extern "C" int kmoe_router_train(const void* x, const int32_t* row_index, int64_t T, int d, const void* w_in,
                                  const void* w_out, int E, const float* logit_bias, int k, float* logits,

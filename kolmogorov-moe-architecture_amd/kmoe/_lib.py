@@ -71,6 +71,9 @@ _SIGNATURES = {
     "kmoe_dequant_rows_fp8": (_i32, [_vp, _vp, _i64, _vp, _i32, _vp, _vp]),
     "kmoe_fake_quant_e4m3_cols": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _vp]),
     "kmoe_router_rms": (_i32, [_vp, _vp, _i64, _i32, _vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _vp, _f32, _vp, _vp]),
+    "kmoe_moe_forward_workspace_bytes": (_sz, [_i64, _i32, _i32, _i32, _i32]),
+    "kmoe_moe_forward": (_i32, [_vp, _i64, _i32, _vp, _vp, _i32, _vp, _i32, _vp, _vp, _i32, _i64, _f32, _vp, _vp, _i32,
+                                _vp, _vp, _f32, _f32, _vp, _sz, _vp]),
     "kmoe_gemm_gate_up_rows_scaled": (_i32, [_vp, _vp, _i64, _vp, _vp, _i32, _i32, _i32, _i64, _vp, _vp, _vp, _vp]),
     "kmoe_combine_residual": (_i32, [_vp, _i32, _vp, _vp, _i32, _vp, _vp, _vp, _i64, _vp, _i32, _vp]),
     "kmoe_combine_residual_dropout": (_i32, [_vp, _i32, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _f32, _i64, _vp, _i32,
@@ -143,7 +146,7 @@ def load():
 
 def call(name: str, *args):
     """Calls a status-returning entry point and raises KmoeError on failure."""
-    lib = load()
+    lib = _LIB or load()
     rc = getattr(lib, name)(*args)
     if rc != KMOE_OK:
         raise KmoeError(name, rc, lib.kmoe_last_error().decode())
@@ -151,10 +154,13 @@ def call(name: str, *args):
 
 
 def ptr(t):
-    """Device pointer of a tensor (None for None)."""
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """Device address of a tensor (None for None), for a void* argument."""
+    return None if t is None else t.data_ptr()
 
 
 def stream_ptr(device=None):
+    """The device's current HIP stream, for a void* argument."""
     import torch
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    if isinstance(device, torch.device) and device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream

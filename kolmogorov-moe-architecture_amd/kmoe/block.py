@@ -184,18 +184,16 @@ class MoEFFNBlock(nn.Module):
         x2d = h.reshape(T, d)
         xb = x2d.to(torch.bfloat16).contiguous()
         w_in_g, w_out, pw = self._fused_weights()
-        router = ffn.router
-        bias = None
-        if router.logit_bias is not None:
-            if router.logit_bias.device != h.device:
-                router.logit_bias = router.logit_bias.to(h.device)
-            bias = router.logit_bias
+        bias = ffn.router.device_bias(xb)
+        keep, keep_scale = self._dropout_keep(T, d, h.device)
+        if keep is None and ffn._one_call(T):
+            return ffn.forward_one_call(xb, w_in_g, w_out, pw, out_dtype, residual=x2d,
+                                        rms_eps=self.ffn_norm.eps).view(B, S, d)
         r = ops.router(xb, w_in_g, w_out, k, bias=bias, rms_eps=self.ffn_norm.eps)
         cap = ops.capacity_of(ffn.capacity_factor, T, k, E) if ffn.drop_overflow else 0
         disp = ops.dispatch(xb, r.idx, r.w, E, capacity=cap, materialize=False)
         hbuf = ops.gemm_gate_up_rows(xb, None, disp.row_token, disp.offsets, pw, T * k, rscale=r.rscale)
         yperm = ops.gemm_down(hbuf, None, disp.offsets, pw, T * k)
-        keep, keep_scale = self._dropout_keep(T, d, h.device)
         y = ops.combine(yperm, disp.slot_row.view(T, k), disp.slot_w.view(T, k), T, out_dtype=out_dtype,
                         residual=x2d, keep_mask=keep, keep_scale=keep_scale)
         ffn._set_token_choice_aux(r, disp, T)

@@ -112,17 +112,19 @@ class Router(_RouterMLP):
         # fp32 per-expert logit bias (kept out of the state dict and of dtype casts)
         self.logit_bias = None if bias is None else torch.tensor(list(bias), dtype=torch.float32)
 
+    def device_bias(self, x2d: torch.Tensor) -> Optional[torch.Tensor]:
+        """The fp32 logit bias on x2d's device, or None."""
+        if self.logit_bias is not None and self.logit_bias.device != x2d.device:
+            self.logit_bias = self.logit_bias.to(x2d.device)
+        return self.logit_bias
+
     def route(self, x2d: torch.Tensor, row_index: Optional[torch.Tensor] = None,
               T: Optional[int] = None, save_hidden: bool = False, hist: bool = True) -> ops.RouterOut:
         """Kernel-level routing of flattened tokens: fp32 logits, int64 idx, f32 weights.
         With moe_balanced_routing the picks are the capacity-balanced assignment
         (moe.py:443-451) over all the tokens of the call."""
         w_in, w_out = self._kernel_weights()
-        bias = None
-        if self.logit_bias is not None:
-            if self.logit_bias.device != x2d.device:
-                self.logit_bias = self.logit_bias.to(x2d.device)
-            bias = self.logit_bias
+        bias = self.device_bias(x2d)
         if self.balanced_routing:
             r = ops.router(x2d, w_in, w_out, 0, bias=bias, row_index=row_index, T=T, save_hidden=save_hidden)
             idx, w = ops.balanced_topk(r.logits, self.top_k)
@@ -736,9 +738,29 @@ class MoELayer(nn.Module):
             self.aux_loss = aux if self.training else 0.0
             return y
         x2d = hidden_states.reshape(B * S, d)
-        y, r, disp = self.forward_rows(x2d, T=B * S, out_dtype=self._out_dtype(hidden_states))
-        self._set_token_choice_aux(r, disp, B * S)
+        if self._one_call(B * S):
+            y = self.forward_one_call(x2d, *self.router._kernel_weights(), self.grouped_experts.packed(),
+                                      self._out_dtype(hidden_states))
+        else:
+            y, r, disp = self.forward_rows(x2d, T=B * S, out_dtype=self._out_dtype(hidden_states))
+            self._set_token_choice_aux(r, disp, B * S)
         return _forward_only(y.view(B, S, d).to(hidden_states.dtype), hidden_states, *self.parameters())
+
+    def _one_call(self, T) -> bool:
+        """Whether a token-choice forward of T tokens without gradients runs as one native
+        call: gated bf16 experts and plain top-k routing, no per-stage timing."""
+        ge = self.grouped_experts
+        return T > 0 and ge.gated and not ge.use_fp8 and not self.router.balanced_routing and not ops.stage_timing()
+
+    def forward_one_call(self, x2d, w_in, w_out, pw, out_dtype, residual=None, rms_eps=None):
+        """ops.moe_forward with this layer's settings; sets last_expert_counts and aux_loss."""
+        T = x2d.shape[0]
+        cap = ops.capacity_of(self.capacity_factor, T, self.top_k, self.n_experts) if self.drop_overflow else 0
+        aux_w = (self.load_balance_loss_weight, self.router_z_loss_weight) if self.training else None
+        y, self.last_expert_counts, aux = ops.moe_forward(x2d, w_in, w_out, self.top_k, self.router.device_bias(x2d), pw,
+                                                          cap, out_dtype, residual=residual, rms_eps=rms_eps, aux=aux_w)
+        self.aux_loss = aux[0] if aux is not None else 0.0
+        return y
 
     def forward_rows(self, x2d, T, row_index=None, T_out=None, out_map=None, scale=None,
                      out_dtype=torch.bfloat16, residual=None):

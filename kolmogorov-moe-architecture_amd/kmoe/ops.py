@@ -41,10 +41,26 @@ def _stream(t):
 _STAGE_EVENTS: Optional[list] = None
 
 
-class _Stage:
+def _Stage(name):
+    """Context of one stage: records its events when a recorder is installed."""
+    return _NO_STAGE if _STAGE_EVENTS is None else _TimedStage(name)
+
+
+class _NoStage:
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        return False
+
+
+_NO_STAGE = _NoStage()
+
+
+class _TimedStage:
     def __init__(self, name):
         self.name = name
-        self.on = _STAGE_EVENTS is not None and (_STAGE_ONLY is None or name in _STAGE_ONLY)
+        self.on = _STAGE_ONLY is None or name in _STAGE_ONLY
 
     def __enter__(self):
         if self.on:
@@ -509,6 +525,52 @@ def combine(yperm, src_row, src_w, T_out, out_map=None, scale=None, out_dtype=_B
         _lib.call("kmoe_combine_residual", ptr(yperm), d, ptr(src_row), ptr(src_w), fan, ptr(out_map), ptr(scale),
                   ptr(residual), T_out, ptr(y), ydt, _stream(yperm))
     return y
+
+
+def stage_timing() -> bool:
+    """Whether a per-stage event recorder is installed."""
+    return _STAGE_EVENTS is not None
+
+
+def moe_forward(x2d, w_in, w_out, k, bias, pw: PackedWeights, capacity, out_dtype, residual=None, rms_eps=None,
+                aux=None):
+    """The token-choice layer forward without gradients in one native call (bf16 gated
+    experts): (y (T, d), counts (E,) int32, aux (3,) f32 or None), the results of router,
+    dispatch, the two expert products and combine.
+    rms_eps: of RMSNorm(x), the norm weight folded into w_in and pw.  aux = (w_lb, w_z): also the
+    aux losses of aux_loss().  residual (T, d): added in the combine."""
+    _need_gpu(x2d, w_in, w_out)
+    x2d = _contig(x2d, _BF16)
+    w_in = _contig(w_in, _BF16)
+    w_out = _contig(w_out, _BF16)
+    T, d = x2d.shape
+    E = w_out.shape[0]
+    if w_in.shape != (_lib.ROUTER_HIDDEN, d) or w_out.shape[1] != _lib.ROUTER_HIDDEN:
+        raise ValueError(f"kmoe.router: weight shapes {tuple(w_in.shape)}, {tuple(w_out.shape)} "
+                         f"do not match d={d}, hidden={_lib.ROUTER_HIDDEN}")
+    if (pw.E, pw.d) != (E, d) or pw.fp8:
+        raise ValueError(f"kmoe.moe_forward: packed weights of {pw.E} experts, d={pw.d} (fp8={pw.fp8}) for a router "
+                         f"of {E} experts, d={d}")
+    dev = x2d.device
+    bias = _contig(bias, torch.float32)
+    y = torch.empty(T, d, device=dev, dtype=out_dtype)
+    if residual is not None:
+        residual = _contig(residual, out_dtype)
+        if residual.shape != (T, d):
+            raise ValueError(f"kmoe.combine: residual shape {tuple(residual.shape)} != {(T, d)}")
+    counts = torch.empty(E, device=dev, dtype=torch.int32)
+    aux_out = None
+    w_lb = w_z = 0.0
+    if aux is not None:
+        w_lb, w_z = aux
+        aux_out = torch.empty(3, device=dev, dtype=torch.float32)
+    wsb = (_lib._LIB or _lib.load()).kmoe_moe_forward_workspace_bytes(T, d, E, k, pw.F)
+    ws = torch.empty(wsb, device=dev, dtype=torch.uint8)
+    _lib.call("kmoe_moe_forward", ptr(x2d), T, d, ptr(w_in), ptr(w_out), E, ptr(bias), k, ptr(pw.w13), ptr(pw.w3), pw.F,
+              int(capacity), -1.0 if rms_eps is None else float(rms_eps), ptr(residual), ptr(y),
+              _lib.DTYPE_F32 if out_dtype == torch.float32 else _lib.DTYPE_BF16, ptr(counts), ptr(aux_out), float(w_lb),
+              float(w_z), ptr(ws), wsb, _stream(x2d))
+    return y, counts, aux_out
 
 
 class ECSelectOut(NamedTuple):

@@ -276,3 +276,40 @@ def test_direct_experts_call_after_drop_layer_drops_nothing(dev):
         W = [f(t) for t in (ge.w1, ge.w2, ge.w3)]
         ref = token_outputs(f(x.view(T, 128)), f(idx), f(w), np.ones((T, 2), bool), W, list(range(T)))
     assert relL2(f(y), ref) <= 1e-2  # every token has both of its experts
+
+
+@pytest.mark.parametrize("T,d,E,k,F,opts", [(1, 256, 4, 2, 352, ""), (33, 128, 8, 1, 128, "bias"), (513, 64, 3, 3, 40, "cap"),
+                                            (700, 320, 16, 4, 136, "cap bias f32"), (8193, 64, 64, 8, 64, "strided"),
+                                            (66000, 64, 4, 2, 64, "")])
+@pytest.mark.parametrize("block", [False, True])
+def test_one_call_forward_matches_separate_launches(dev, T, d, E, k, F, opts, block):
+    """The layer's (and the fused block's) forward as one native call gives the bits of the
+    separate entry points (which run while a per-stage recorder is installed): output, aux
+    loss and routed counts, with a logit bias, the capacity drop, f32 input, a strided
+    input, both router tiles and dispatch scans (1024 blocks of 64 tokens at 65536)."""
+    from kmoe import ops
+    from kmoe.block import MoEFFNBlock
+    from kmoe.config import AdvancedMoEConfig
+    from kmoe.moe import MoELayer
+
+    cfg = AdvancedMoEConfig(d_model=d, n_experts=E, moe_top_k=k, d_ff_expert=F, moe_drop_overflow="cap" in opts,
+                            moe_capacity_factor=1.0, residual_dropout=0.0, mod_enabled=False,
+                            moe_router_bias=[0.1 * e for e in range(E)] if "bias" in opts else None)
+    dt = torch.float32 if "f32" in opts else torch.bfloat16
+    torch.manual_seed(T)
+    m = (MoEFFNBlock(cfg) if block else MoELayer(cfg)).to(dev, dt).train()
+    x = torch.randn(1, T, 2 * d if "strided" in opts else d, device=dev, dtype=dt)[..., :d]
+    layer = m.ffn if block else m
+    outs = []
+    with torch.no_grad():
+        for events in (None, []):
+            ops.set_stage_timing(events)
+            try:
+                y = m(x)
+            finally:
+                ops.set_stage_timing(None)
+            outs.append((y, layer.aux_loss, layer.last_expert_counts))
+    torch.cuda.synchronize()
+    assert events, "the second pass runs the separate entry points"
+    for a, b in zip(*outs):
+        assert a.dtype == b.dtype and torch.equal(a, b)
