@@ -186,16 +186,26 @@ __device__ __forceinline__ void wgrad_tn_tile(const GemmArgs& g, uint8_t* lds, i
   // ---- epilogue: acc[mb][nb][t] is row wm*128 + mb*16 + l%16, column wn*128 + nb*16 +
   // 4 (l/16) + t of the tile
   if constexpr (OUT == OUT_F32) {
+    // a lane's four columns as one 16-byte store (n_valid and ldc are multiples of 8), where
+    // the buffer is aligned for it
+    const bool vec = (reinterpret_cast<uintptr_t>(g.Cf) & 15) == 0;
 #pragma unroll
-    for (int mb = 0; mb < 8; ++mb)
+    for (int mb = 0; mb < 8; ++mb) {
+      const int row = m0 + wm * 128 + mb * 16 + i16;
+      if (row >= M) continue;
 #pragma unroll
-      for (int nb = 0; nb < 8; ++nb)
+      for (int nb = 0; nb < 8; ++nb) {
+        const int col = n0 + wn * 128 + nb * 16 + 4 * kq;
+        if (col >= g.n_valid) continue;
+        float* const p = g.Cf + (int64_t)row * g.ldc + col;
+        if (vec) {
+          *reinterpret_cast<f32x4_t*>(p) = acc[mb][nb];
+        } else {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int row = m0 + wm * 128 + mb * 16 + i16;
-          const int col = n0 + wn * 128 + nb * 16 + 4 * kq + t;
-          if (row < M && col < g.n_valid) g.Cf[(int64_t)row * g.ldc + col] = acc[mb][nb][t];
+          for (int t = 0; t < 4; ++t) p[t] = acc[mb][nb][t];
         }
+      }
+    }
   } else {
     // bf16 through LDS (rows padded by 16 bytes): a lane's four columns as 8 bytes, then
     // 16-byte row stores
@@ -211,18 +221,29 @@ __device__ __forceinline__ void wgrad_tn_tile(const GemmArgs& g, uint8_t* lds, i
         *reinterpret_cast<i32x2_t*>(wbase + mb * 16 * OSTR + nb * 32) = i32x2_t{(int)lo, (int)hi};
       }
     __syncthreads();
-    for (int c = tid; c < BM * 32; c += GEMM_THREADS) {
-      const int trow = c >> 5, tc = (c & 31) * 8;  // tile row, first column of the 8
-      const int grow = m0 + trow;
-      uint16_t* base = g.C;
-      int gcol = n0 + tc;
-      if constexpr (OUT == OUT_SPLIT) {
-        base = tc < 128 ? g.C : g.C2;
-        gcol = nt * 128 + (tc & 127);
+    // a thread stores the same 16-byte chunk of every eighth row; eight LDS reads go out
+    // ahead of their stores (one read, wait, store at a time serialised the loop on the LDS
+    // latency: dW1|dW2 of 8192 rows over 16 experts, d 2048, F 2816, 340 -> 332 us)
+    const int tc = (tid & 31) * 8, tr0 = tid >> 5;
+    uint16_t* base = g.C;
+    int gcol = n0 + tc;
+    if constexpr (OUT == OUT_SPLIT) {
+      base = tc < 128 ? g.C : g.C2;
+      gcol = nt * 128 + (tc & 127);
+    }
+    if (gcol < g.n_valid) {
+      uint16_t* const gp = base + (int64_t)(m0 + tr0) * g.ldc + gcol;
+      const uint8_t* const lp = lds + tr0 * OSTR + tc * 2;
+      const int rows = M - m0 - tr0;
+#pragma unroll
+      for (int h = 0; h < BM / 8; h += 8) {
+        i32x4_t v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const i32x4_t*>(lp + (h + u) * 8 * OSTR);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if ((h + u) * 8 < rows) *reinterpret_cast<i32x4_t*>(gp + (int64_t)(h + u) * 8 * g.ldc) = v[u];
       }
-      if (grow < M && gcol < g.n_valid)
-        *reinterpret_cast<i32x4_t*>(base + (int64_t)grow * g.ldc + gcol) =
-            *reinterpret_cast<const i32x4_t*>(lds + trow * OSTR + tc * 2);
     }
   }
 }

@@ -26,7 +26,9 @@ from . import _lib, ops
 from ._lib import ptr
 
 _BF16 = torch.bfloat16
-WG_SPLIT = 512  # token rows per split-K segment of the router's weight gradient
+# token rows per split-K segment of the router's weight gradient (128 x d outputs are few
+# tiles: at 4096 tokens, d 2048, segments of 512 rows made 64 workgroups, of 128 rows 256)
+WG_SPLIT = 128
 
 
 def _ru(a: int, b: int) -> int:
