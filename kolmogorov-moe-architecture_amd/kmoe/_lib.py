@@ -15,6 +15,7 @@ LIB_PATH = os.path.join(_HERE, "libkmoe.so")
 HEADER_PATH = os.path.abspath(os.path.join(_HERE, "..", "..", "include", "kmoe.h"))
 
 KMOE_OK = 0
+KMOE_ERR_SHAPE = -2
 DTYPE_BF16 = 0
 DTYPE_F32 = 1
 DTYPE_FP8_E4M3 = 2

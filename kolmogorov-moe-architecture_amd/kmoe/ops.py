@@ -551,6 +551,8 @@ def moe_forward(x2d, w_in, w_out, k, bias, pw: PackedWeights, capacity, out_dtyp
     if (pw.E, pw.d) != (E, d) or pw.fp8:
         raise ValueError(f"kmoe.moe_forward: packed weights of {pw.E} experts, d={pw.d} (fp8={pw.fp8}) for a router "
                          f"of {E} experts, d={d}")
+    if rms_eps is not None and not rms_eps >= 0.0:  # negative means "no norm" to the native call
+        raise _lib.KmoeError("kmoe_moe_forward", _lib.KMOE_ERR_SHAPE, f"rms_eps {rms_eps} must be >= 0")
     dev = x2d.device
     bias = _contig(bias, torch.float32)
     y = torch.empty(T, d, device=dev, dtype=out_dtype)

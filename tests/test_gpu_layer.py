@@ -313,3 +313,16 @@ def test_one_call_forward_matches_separate_launches(dev, T, d, E, k, F, opts, bl
     assert events, "the second pass runs the separate entry points"
     for a, b in zip(*outs):
         assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("eps", [-1e-5, float("nan")])
+def test_one_call_forward_refuses_eps(dev, eps):
+    """A fused block with a negative or NaN norm eps raises, as the router entry point of the
+    separate launches does (the native call takes a negative value as "no norm")."""
+    import kmoe
+    from kmoe.config import AdvancedMoEConfig
+
+    m = kmoe.MoEFFNBlock(AdvancedMoEConfig(d_model=64, n_experts=2, moe_top_k=1, d_ff_expert=64, residual_dropout=0.0,
+                                           mod_enabled=False, norm_eps=eps)).to(dev, torch.bfloat16).eval()
+    with torch.no_grad(), pytest.raises(kmoe.KmoeError):
+        m(torch.randn(1, 4, 64, device=dev, dtype=torch.bfloat16))
