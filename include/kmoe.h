@@ -352,6 +352,14 @@ int kmoe_pack_weights_bwd(const void* w1, const void* w2, const void* w3, int w_
 int kmoe_gemm_grouped(const void* a, const int32_t* offsets, int E, int K, int64_t max_rows, const void* b_packed,
                       int64_t b_expert_rows, int N, void* c, int64_t ldc, int n_valid, void* stream);
 
+/* kmoe_gemm_grouped with the weights as they are, not packed: b (E, N, K) bf16, contiguous,
+ * 16-byte aligned, N % 256 == 0.  With b2, b and b2 are (E, N, K/2) and their columns are
+ * taken interleaved per 128 (K % 256 == 0).  The products and their order of sums are those
+ * on the packed copies.
+ * dh = dyperm . w3^T: b = w3 (E, F, d);  dx = dgu . [w1|w2]^T: b = w1, b2 = w2 (E, d, F). */
+int kmoe_gemm_grouped_weights(const void* a, const int32_t* offsets, int E, int K, int64_t max_rows, const void* b,
+                              const void* b2, int N, void* c, int64_t ldc, void* stream);
+
 /* SwiGLU backward on the packed order: s = sigmoid(g),
  *   dg = dh * u * s * (1 + g (1 - s)),  du = dh * g * s
  * dh (rows, F_pad), gu / dgu (rows, 2*F_pad) bf16; rows < *n_rows_dev if given. */

@@ -35,7 +35,8 @@ bool small_rows_product(bool gate_up, int E, int64_t max_rows, int64_t b_expert_
 int launch_gemm(bool gate_up, bool fp8, const void* A, const float* a_scale, const int32_t* row_token,
                 const int32_t* row_index, int64_t n_a_rows, const int32_t* offsets, int E, int K, int64_t max_rows,
                 const void* B, int64_t b_expert_rows, const float* b_scale, void* C, int64_t ldc, int n_valid,
-                int n_tiles, hipStream_t s, void* C2 = nullptr, void* gu_out = nullptr) {
+                int n_tiles, hipStream_t s, void* C2 = nullptr, void* gu_out = nullptr, int64_t ldb_bytes = 0,
+                const void* B2 = nullptr) {
   const int eb = fp8 ? 1 : 2;
   const int64_t slots = kmoe::ceil_div<int64_t>(max_rows, BM) + E;
   // every tile of the worst-case slot count, plus one narrow tile per resident
@@ -60,7 +61,8 @@ int launch_gemm(bool gate_up, bool fp8, const void* A, const float* a_scale, con
   g.row_index = row_index;
   g.B = static_cast<const uint8_t*>(B);
   g.b_expert_rows = b_expert_rows;
-  g.ldb_bytes = kbytes + WPAD;
+  g.B2 = static_cast<const uint8_t*>(B2);
+  g.ldb_bytes = ldb_bytes ? ldb_bytes : kbytes + WPAD;
   g.b_scale = b_scale;
   g.k_bytes = kbytes;
   g.C = static_cast<uint16_t*>(C);
@@ -80,7 +82,9 @@ int launch_gemm(bool gate_up, bool fp8, const void* A, const float* a_scale, con
   if (!fp8 && small_rows_product(gate_up, E, max_rows, b_expert_rows, g.ldb_bytes, n_tiles)) {
     const int n_ct = n_tiles * (gate_up ? BN / 2 : BN) / small_cols(gate_up);
     launch_small_rows(GemmLaunch{g, offsets, E, n_ct, n_cu, (unsigned)(small_slots(E, max_rows) * n_ct), s}, gate_up);
-  } else if (fp8)
+  } else if (B2)
+    launch_dual(l);
+  else if (fp8)
     launch_fp8(l, gate_up, gu_out != nullptr);
   else if (row_token && gu_out)
     launch_gate_up_rows_gu(l);
@@ -231,4 +235,21 @@ extern "C" int kmoe_gemm_grouped(const void* a, const int32_t* offsets, int E, i
                              kmoe::as_stream(stream));
   if (rc) return rc;
   return kmoe::check_launch("kmoe_gemm_grouped");
+}
+
+extern "C" int kmoe_gemm_grouped_weights(const void* a, const int32_t* offsets, int E, int K, int64_t max_rows,
+                                         const void* b, const void* b2, int N, void* c, int64_t ldc, void* stream) {
+  KMOE_REQUIRE(a && offsets && b && c, KMOE_ERR_NULL, "kmoe_gemm_grouped_weights: null buffer");
+  KMOE_REQUIRE(E >= 1 && E <= KMOE_MAX_EXPERTS, KMOE_ERR_SHAPE, "kmoe_gemm_grouped_weights: E=%d out of range", E);
+  // whole tiles of weight rows and of columns: nothing past a matrix's end is read
+  KMOE_REQUIRE(K > 0 && K % (b2 ? 256 : 64) == 0 && N > 0 && N % BN == 0 && N <= ldc, KMOE_ERR_SHAPE,
+               "kmoe_gemm_grouped_weights: K=%d, N=%d, ldc=%lld", K, N, (long long)ldc);
+  KMOE_REQUIRE(((reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(b2)) & 15) == 0, KMOE_ERR_SHAPE,
+               "kmoe_gemm_grouped_weights: weights not aligned to 16 bytes");
+  KMOE_REQUIRE(max_rows >= 0 && max_rows < ((int64_t)1 << 31), KMOE_ERR_SHAPE, "kmoe_gemm_grouped_weights: max_rows");
+  if (max_rows == 0) return KMOE_OK;
+  const int rc = launch_gemm(false, false, a, nullptr, nullptr, nullptr, 0, offsets, E, K, max_rows, b, N, nullptr, c,
+                             ldc, N, N / BN, kmoe::as_stream(stream), nullptr, nullptr, (int64_t)K * (b2 ? 1 : 2), b2);
+  if (rc) return rc;
+  return kmoe::check_launch("kmoe_gemm_grouped_weights");
 }

@@ -87,7 +87,7 @@ __device__ __forceinline__ void put_gate_up(const GemmArgs& g, int row, int f, f
 // 256-row tiles 84.5).  Interleaving the waves' steps, eight waves per workgroup and
 // non-temporal weight loads were slower too.
 constexpr int DEPTH = 2;
-template <bool GATE_UP, bool GATHER, bool SAVE_GU, bool RSCALE>
+template <bool GATE_UP, bool GATHER, bool SAVE_GU, bool RSCALE, bool DUAL>
 __global__ __launch_bounds__(256) void small_rows_kernel(GemmArgs g, const int32_t* __restrict__ offsets, int E, int n_ct) {
   __shared__ f32x4_t red[4][4][64];
   const int slot = blockIdx.x / n_ct, ct = blockIdx.x - slot * n_ct;
@@ -101,6 +101,7 @@ __global__ __launch_bounds__(256) void small_rows_kernel(GemmArgs g, const int32
   const int s0 = wave * nk / 4, s1 = (wave + 1) * nk / 4;
 
   const uint8_t* const bbase = g.B + (int64_t)e * g.b_expert_rows * g.ldb_bytes;
+  const uint8_t* const b2base = DUAL ? g.B2 + (int64_t)e * g.b_expert_rows * g.ldb_bytes : nullptr;
   const uint8_t* const abase = GATHER ? g.A : g.A + (int64_t)m0 * g.lda_bytes;
   uint32_t boff[2];
 #pragma unroll
@@ -119,11 +120,13 @@ __global__ __launch_bounds__(256) void small_rows_kernel(GemmArgs g, const int32
     bf16x8_t b[DEPTH][2][2], a[DEPTH][2][MB];
     // step s into ring entry u; steps past the wave's range read nothing (empty window)
     auto load_b = [&](int u, int s) {
-      const __amdgpu_buffer_rsrc_t rs = make_rsrc_window(bbase, s < s1 ? 0x7fffffff : 0);
+      const uint8_t* const base = DUAL && dual_step_second(s) ? b2base : bbase;
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc_window(base, s < s1 ? 0x7fffffff : 0);
+      const int soff = DUAL ? dual_step_offset(s) : s * KB;
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) b[u][i][j] = load_frag(rs, boff[j] + 64u * i, s * KB);
+        for (int i = 0; i < 2; ++i) b[u][i][j] = load_frag(rs, boff[j] + 64u * i, soff);
     };
     uint32_t aoff[MB];
     auto load_a = [&](int u, int s) {
@@ -187,9 +190,9 @@ __global__ __launch_bounds__(256) void small_rows_kernel(GemmArgs g, const int32
   }
 }
 
-template <bool GATE_UP, bool GATHER, bool SAVE_GU, bool RSCALE>
+template <bool GATE_UP, bool GATHER, bool SAVE_GU, bool RSCALE, bool DUAL = false>
 void launch_small(const GemmLaunch& l) {
-  hipLaunchKernelGGL((small_rows_kernel<GATE_UP, GATHER, SAVE_GU, RSCALE>), dim3(l.blocks), dim3(256), 0, l.s, l.g,
+  hipLaunchKernelGGL((small_rows_kernel<GATE_UP, GATHER, SAVE_GU, RSCALE, DUAL>), dim3(l.blocks), dim3(256), 0, l.s, l.g,
                      l.offsets, l.E, l.n_tiles);
 }
 
@@ -198,7 +201,9 @@ void launch_small(const GemmLaunch& l) {
 namespace kmoe_tiles {
 
 void launch_small_rows(const GemmLaunch& l, bool gate_up) {
-  if (!gate_up)
+  if (l.g.B2)
+    launch_small<false, false, false, false, true>(l);
+  else if (!gate_up)
     launch_small<false, false, false, false>(l);
   else if (!l.g.row_token)
     launch_small<true, false, false, false>(l);

@@ -276,6 +276,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc_window(const void* b
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, n, 0x00020000);
 }
 
+// DUAL products (dx = dg . w1^T + du . w2^T with [dg | du] interleaved per 128 columns, read
+// from w1 and w2 (E, d, F) as they are): of four K-steps of 64, the first two are 128
+// columns of B, the other two the same columns of B2.
+__device__ __forceinline__ bool dual_step_second(int ks) { return ks & 2; }
+__device__ __forceinline__ int dual_step_offset(int ks) { return (ks >> 2) * 2 * KB + (ks & 1) * KB; }
+
 struct GemmArgs {
   const uint8_t* A;
   int64_t lda_bytes;
@@ -283,6 +289,7 @@ struct GemmArgs {
   const int32_t* row_token;
   const int32_t* row_index;
   const uint8_t* B;
+  const uint8_t* B2;  // DUAL tiles: the second weight matrix
   int64_t b_expert_rows;
   int64_t ldb_bytes;
   const float* b_scale;
@@ -349,7 +356,9 @@ constexpr int OUT_BF16 = 0, OUT_SPLIT = 1, OUT_F32 = 2;
 // run with NMA < 4 (the first NMA blocks), which skips the other blocks' fragment
 // reads, MFMAs and epilogue (their accumulators stay 0 and are never stored).  The
 // waves of a workgroup may differ in NMA: loads, LDS writes and barriers are the same.
-template <bool GATE_UP, bool FP8, bool GATHER, int WNB, bool SAVE_GU = false, bool RSCALE = false, int NMA = 4>
+// DUAL: see dual_step.
+template <bool GATE_UP, bool FP8, bool GATHER, int WNB, bool SAVE_GU = false, bool RSCALE = false, int NMA = 4,
+          bool DUAL = false>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, uint8_t* lds, int e, int m0, int m_end, int nt,
                                           int q) {
   static_assert(WNB == 4 || WNB == 2 || WNB == 1, "tile width");
@@ -374,7 +383,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, uint8_t* lds, int e
 
   const int64_t brow0 = (int64_t)e * g.b_expert_rows + (int64_t)nt * BN;  // full packed tile
   const __amdgpu_buffer_rsrc_t arsrc = make_rsrc(GATHER ? g.A : g.A + (int64_t)m0 * g.lda_bytes);
-  const __amdgpu_buffer_rsrc_t brsrc = make_rsrc(g.B + brow0 * g.ldb_bytes);
+  const uint8_t* const bbase = g.B + brow0 * g.ldb_bytes;
+  const uint8_t* const b2base = DUAL ? g.B2 + brow0 * g.ldb_bytes : nullptr;
+  const __amdgpu_buffer_rsrc_t brsrc = make_rsrc(bbase);
   const int nk = g.k_bytes / KB;
   // LDS stage s: [A tile | B tile]
   auto la_buf = [&](int st) { return lds + st * (TB + TBB); };
@@ -449,6 +460,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, uint8_t* lds, int e
     const int ks = kt < nk ? kt : nk - 1;
     if (qq < BLK_PER_WAVE)
       stg[qq] = __builtin_amdgcn_raw_buffer_load_b128(arsrc, a_off[qq], ks * KB, 0);
+    else if constexpr (DUAL)
+      stg[qq] = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(dual_step_second(ks) ? b2base : bbase),
+                                                      b_off[qq - BLK_PER_WAVE], dual_step_offset(ks), 0);
     else
       stg[qq] = __builtin_amdgcn_raw_buffer_load_b128(brsrc, b_off[qq - BLK_PER_WAVE], ks * KB, 0);
   };
@@ -1214,7 +1228,7 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
 // e4m3 products of at least two K-steps: the full rounds (and whole tail tiles) go to
 // gemm_full_tiles on the first n_cu workgroups, the narrow tiles to the ones after them (a
 // single K-step: all tiles in halves).
-template <bool GATE_UP, bool FP8, bool GATHER, bool SAVE_GU = false, bool RSCALE = false>
+template <bool GATE_UP, bool FP8, bool GATHER, bool SAVE_GU = false, bool RSCALE = false, bool DUAL = false>
 __global__ __launch_bounds__(GEMM_THREADS, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void grouped_gemm_kernel(
     GemmArgs g, const int32_t* __restrict__ offsets, int E, int n_tiles, int n_cu) {
   static_assert(!(GATHER && FP8), "the fp8 path reads rows quantised by the dispatch");
@@ -1268,17 +1282,17 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) __attribute__((amdgpu_waves_per_eu
       // row blocks of this wave holding rows (wave-uniform): 4 (more than 64 rows), 2, 1, 0
       const int wrows = m_end - m0 - (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >> 1) * 128;
       if (wrows > 64)
-        gemm_tile<GATE_UP, FP8, GATHER, 4, SAVE_GU, RSCALE, 4>(g, lds, e, m0, m_end, nt, 0);
+        gemm_tile<GATE_UP, FP8, GATHER, 4, SAVE_GU, RSCALE, 4, DUAL>(g, lds, e, m0, m_end, nt, 0);
       else if (wrows > 32)
-        gemm_tile<GATE_UP, FP8, GATHER, 4, SAVE_GU, RSCALE, 2>(g, lds, e, m0, m_end, nt, 0);
+        gemm_tile<GATE_UP, FP8, GATHER, 4, SAVE_GU, RSCALE, 2, DUAL>(g, lds, e, m0, m_end, nt, 0);
       else if (wrows > 0)
-        gemm_tile<GATE_UP, FP8, GATHER, 4, SAVE_GU, RSCALE, 1>(g, lds, e, m0, m_end, nt, 0);
+        gemm_tile<GATE_UP, FP8, GATHER, 4, SAVE_GU, RSCALE, 1, DUAL>(g, lds, e, m0, m_end, nt, 0);
       else
-        gemm_tile<GATE_UP, FP8, GATHER, 4, SAVE_GU, RSCALE, 0>(g, lds, e, m0, m_end, nt, 0);
+        gemm_tile<GATE_UP, FP8, GATHER, 4, SAVE_GU, RSCALE, 0, DUAL>(g, lds, e, m0, m_end, nt, 0);
     } else if (split == 2)
-      gemm_tile<GATE_UP, FP8, GATHER, 2, SAVE_GU, RSCALE>(g, lds, e, m0, m_end, nt, q);
+      gemm_tile<GATE_UP, FP8, GATHER, 2, SAVE_GU, RSCALE, 4, DUAL>(g, lds, e, m0, m_end, nt, q);
     else
-      gemm_tile<GATE_UP, FP8, GATHER, 1, SAVE_GU, RSCALE>(g, lds, e, m0, m_end, nt, q);
+      gemm_tile<GATE_UP, FP8, GATHER, 1, SAVE_GU, RSCALE, 4, DUAL>(g, lds, e, m0, m_end, nt, q);
   }
 }
 
@@ -1291,14 +1305,15 @@ struct GemmLaunch {
   unsigned blocks;
   hipStream_t s;
 };
-template <bool GATE_UP, bool FP8, bool GATHER, bool SAVE_GU = false, bool RSCALE = false>
+template <bool GATE_UP, bool FP8, bool GATHER, bool SAVE_GU = false, bool RSCALE = false, bool DUAL = false>
 void launch_variant(const GemmLaunch& l) {
-  hipLaunchKernelGGL((grouped_gemm_kernel<GATE_UP, FP8, GATHER, SAVE_GU, RSCALE>), dim3(l.blocks), dim3(GEMM_THREADS), 0,
-                     l.s, l.g, l.offsets, l.E, l.n_tiles, l.n_cu);
+  hipLaunchKernelGGL((grouped_gemm_kernel<GATE_UP, FP8, GATHER, SAVE_GU, RSCALE, DUAL>), dim3(l.blocks),
+                     dim3(GEMM_THREADS), 0, l.s, l.g, l.offsets, l.E, l.n_tiles, l.n_cu);
 }
 void launch_gate_up_rows(const GemmLaunch& l);                    // bf16, gathered rows (RSCALE with a_scale)
 void launch_gate_up_rows_gu(const GemmLaunch& l);                 // the same, saving the gate / up values
 void launch_permuted(const GemmLaunch& l, bool gate_up);          // bf16, permuted rows
+void launch_dual(const GemmLaunch& l);                            // the same, no gate/up, weights from B and B2
 void launch_fp8(const GemmLaunch& l, bool gate_up, bool save_gu); // e4m3, permuted rows
 // bf16, few rows per expert (kmoe_gemm_small.hip): slots of SMALL_ROWS rows, n_tiles column
 // tiles of small_cols() output columns

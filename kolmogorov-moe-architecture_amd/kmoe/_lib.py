@@ -95,6 +95,7 @@ _SIGNATURES = {
     "kmoe_pack_weights_plain_bwd": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _vp, _vp, _vp]),
     "kmoe_silu_rows": (_i32, [_vp, _i64, _vp, _i32, _vp, _vp]),
     "kmoe_silu_bwd": (_i32, [_vp, _vp, _i64, _vp, _i32, _vp, _vp]),
+    "kmoe_gemm_grouped_weights": (_i32, [_vp, _vp, _i32, _i32, _i64, _vp, _vp, _i32, _vp, _i64, _vp]),
     "kmoe_gemm_grouped": (_i32, [_vp, _vp, _i32, _i32, _i64, _vp, _i64, _i32, _vp, _i64, _i32, _vp]),
     "kmoe_swiglu_bwd": (_i32, [_vp, _vp, _i64, _vp, _i32, _vp, _vp]),
     "kmoe_reduce_f32": (_i32, [_vp, _i64, _i64, _vp, _i32, _vp]),

@@ -9,9 +9,9 @@ its native grouped kernel has no backward at all (moe_arch/kernels/__init__.py:
 
 Data flow (A = routed rows, grouped by expert):
   dy --combine_bwd--> dyperm (A,d), dw (T,k)
-  dh  = dyperm . w3^T            grouped GEMM (packed w3n)
+  dh  = dyperm . w3^T            grouped GEMM (packed w3n, or w3 itself)
   dgu = swiglu_bwd(dh, g, u)     g, u saved by the forward's gate/up GEMM
-  dxp = dgu . [w1|w2]^T          grouped GEMM (packed w13t)
+  dxp = dgu . [w1|w2]^T          grouped GEMM (packed w13t, or w1 and w2 themselves)
   dx  = sum_j dxp[slot(t,j)] + (da . w_in)[t]   (one unit-weight gather of both)
   dW3 = h^T dyperm, dW1|dW2 = xperm^T dgu       per-expert GEMMs on the row buffers (LDS transpose reads)
   dlogits = topk-renorm backward(dw) + aux backward;  da, dW_out (router MLP);  dW_in = da^T x
@@ -36,18 +36,36 @@ def _ru(a: int, b: int) -> int:
 
 
 class BwdWeights(NamedTuple):
-    w3n: torch.Tensor    # (E, round_up(F,256), d) packed rows of w3 (non-gated: of w2)
-    w13t: torch.Tensor   # (E, round_up(d,256), 2*F_pad) packed rows of w1|w2 (non-gated: rows of w1, F_pad)
+    w3n: torch.Tensor    # (E, round_up(F,256), d) packed rows of w3 (non-gated: of w2), or w3 itself (bf16)
+    w13t: torch.Tensor   # (E, round_up(d,256), 2*F_pad) packed rows of w1|w2 (non-gated: rows of w1, F_pad),
+                         # or w1 itself (bf16)
     w_in_t: torch.Tensor  # (round_up(d,256), 128) packed rows of w_in^T
     plain: bool = False  # non-gated experts (silu(x w1) w2)
+    w2: Optional[torch.Tensor] = None  # with w1 itself: w2
+
+
+def _as_they_are(*ws) -> bool:
+    """Whether the backward products read the expert weights w1, w2(, w3) in place of packed
+    copies: bf16, contiguous, and d and F multiples of the 256-row tile (nothing past a
+    matrix's end is read).  New weights, as in every optimizer step, then cost no packs (4096
+    tokens, d 2048, 16 experts, F 2816: 207 us of a 2009 us step); the products themselves take
+    as long within 2% (2042 tokens: 271 us packed, 275 in place)."""
+    return all(w.dtype == _BF16 and w.is_contiguous() and w.data_ptr() % 16 == 0 and w.shape[1] % 256 == 0
+               and w.shape[2] % 256 == 0 for w in ws)
 
 
 def pack_bwd_weights(w1, w2, w3, w_in) -> BwdWeights:
     """Backward packed layouts of the expert weights (w1/w2/w3; w1 None: skipped; w3 None:
     the non-gated experts' w1 (E,d,F), w2 (E,F,d)) and of the router's w_in (None: skipped)."""
     lib = _lib.load()
-    w3n = w13t = wit = None
+    w3n = w13t = wit = second = None
     plain = False
+    if w1 is not None and _as_they_are(*(w for w in (w1, w2, w3) if w is not None)):
+        plain = w3 is None
+        w13t = w1.detach()
+        w3n = (w2 if plain else w3).detach()
+        second = None if plain else w2.detach()
+        w1 = None
     if w1 is not None and w3 is None:
         E, d, F = w1.shape
         dt = w1.dtype if w1.dtype in (torch.float32, _BF16) else torch.float32
@@ -78,7 +96,7 @@ def pack_bwd_weights(w1, w2, w3, w_in) -> BwdWeights:
         wdt = _lib.DTYPE_F32 if dt == torch.float32 else _lib.DTYPE_BF16
         wit = torch.empty(lib.kmoe_packed_w_in_t_bytes(d), device=w_in.device, dtype=torch.uint8)
         _lib.call("kmoe_pack_w_in_t", ptr(w_in), wdt, d, ptr(wit), ops._stream(w_in))
-    return BwdWeights(w3n, w13t, wit, plain)
+    return BwdWeights(w3n, w13t, wit, plain, second)
 
 
 class Saved(NamedTuple):
@@ -158,8 +176,11 @@ def _experts_core(dy, yperm, gu, slot_row, slot_w, kk, offsets, A, bw: BwdWeight
                       ptr(row_index), ptr(scale), ptr(dyperm), ptr(dw), ptr(dscale), s)
     dh = torch.empty(max(A, 1), Fp, device=dev, dtype=_BF16)
     with _stage("bwd_gemm_dh"):
-        _lib.call("kmoe_gemm_grouped", ptr(dyperm), ptr(offsets), E, d, A, ptr(bw.w3n), _ru(F, 256), Fp,
-                  ptr(dh), Fp, Fp, s)
+        if bw.w3n.dtype == _BF16:
+            _lib.call("kmoe_gemm_grouped_weights", ptr(dyperm), ptr(offsets), E, d, A, ptr(bw.w3n), None, F, ptr(dh), F, s)
+        else:
+            _lib.call("kmoe_gemm_grouped", ptr(dyperm), ptr(offsets), E, d, A, ptr(bw.w3n), _ru(F, 256), Fp,
+                      ptr(dh), Fp, Fp, s)
     # gated: [dg | du] from the saved gate / up values; non-gated: dp from the saved p
     kk2 = 1 if bw.plain else 2
     dgu = torch.empty(max(A, 1), kk2 * Fp, device=dev, dtype=_BF16)
@@ -170,8 +191,12 @@ def _experts_core(dy, yperm, gu, slot_row, slot_w, kk, offsets, A, bw: BwdWeight
             _lib.call("kmoe_swiglu_bwd", ptr(dh), ptr(gu), A, ptr(offsets[E:]), F, ptr(dgu), s)
     dxp = torch.empty(A + extra_rows, d, device=dev, dtype=_BF16)
     with _stage("bwd_gemm_dx"):
-        _lib.call("kmoe_gemm_grouped", ptr(dgu), ptr(offsets), E, kk2 * Fp, A, ptr(bw.w13t), _ru(d, 256), d,
-                  ptr(dxp), d, d, s)
+        if bw.w13t.dtype == _BF16:
+            _lib.call("kmoe_gemm_grouped_weights", ptr(dgu), ptr(offsets), E, kk2 * F, A, ptr(bw.w13t), ptr(bw.w2), d,
+                      ptr(dxp), d, s)
+        else:
+            _lib.call("kmoe_gemm_grouped", ptr(dgu), ptr(offsets), E, kk2 * Fp, A, ptr(bw.w13t), _ru(d, 256), d,
+                      ptr(dxp), d, d, s)
     return dxp, dw, dyperm, dgu, dscale
 
 

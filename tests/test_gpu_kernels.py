@@ -806,3 +806,50 @@ def test_small_rows(dev, path, d, F, counts):
                 n = min(128, F - f)
                 assert rel(gu[s:t, 2 * f:2 * f + n], gg[:, f:f + n]) <= 4e-3
                 assert rel(gu[s:t, 2 * f + 128:2 * f + 128 + n], uu[:, f:f + n]) <= 4e-3
+
+
+# ------------------------------------------------------------------ weights read in place
+@pytest.mark.parametrize("d,F,counts", [(256, 256, [1, 0, 2]), (512, 768, [33, 0, 17, 5]), (512, 768, [1500, 17, 0, 2513]),
+                                        (256, 1280, [257] * 40), (2048, 256, [600, 1])])
+@pytest.mark.parametrize("gated", [True, False])
+def test_backward_products_weights_in_place(dev, d, F, counts, gated):
+    """The backward products on bf16 weights as they are give the bits of the products on the
+    packed copies (packed from the same values in f32), on the small-row kernel, full, split
+    and partly empty tiles; and dx against fp32 matmuls (bar 4e-3 rel-L2: one bf16 rounding)."""
+    from kmoe import _lib, backward as BW
+
+    E, A = len(counts), sum(counts)
+    off_l = np.concatenate([[0], np.cumsum(counts)])
+    off = torch.tensor(off_l, dtype=torch.int32, device=dev)
+    g = torch.Generator(device=dev).manual_seed(d + F)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    w1, w2, w3 = (bf16(rnd(*s) * s[2] ** -0.5) for s in ((E, d, F), (E, d, F), (E, F, d)))
+    ws = (w1, w2, w3) if gated else (w1, w3, None)
+    here = BW.pack_bwd_weights(*ws, None)
+    packed = BW.pack_bwd_weights(*(None if w is None else w.float() for w in ws), None)
+    assert here.w13t.data_ptr() == w1.data_ptr() and packed.w13t.dtype == torch.uint8
+    dyp, dgu = bf16(rnd(A, d)), bf16(rnd(A, (2 if gated else 1) * F))
+    s = ops._stream(dyp)
+    p = _lib.ptr
+    outs = []
+    for bw in (here, packed):
+        dh, dx = torch.empty(A, F, device=dev, dtype=torch.bfloat16), torch.empty_like(dyp)
+        if bw is here:
+            _lib.call("kmoe_gemm_grouped_weights", p(dyp), p(off), E, d, A, p(bw.w3n), None, F, p(dh), F, s)
+            _lib.call("kmoe_gemm_grouped_weights", p(dgu), p(off), E, dgu.shape[1], A, p(bw.w13t), p(bw.w2), d, p(dx), d, s)
+        else:
+            _lib.call("kmoe_gemm_grouped", p(dyp), p(off), E, d, A, p(bw.w3n), F, F, p(dh), F, F, s)
+            _lib.call("kmoe_gemm_grouped", p(dgu), p(off), E, dgu.shape[1], A, p(bw.w13t), d, d, p(dx), d, d, s)
+        outs.append((dh, dx))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    for e in range(E):
+        a, b = int(off_l[e]), int(off_l[e + 1])
+        if a == b:
+            continue
+        r = dgu[a:b].float()
+        if gated:
+            r = r.view(b - a, F // 128, 2, 128)
+            ref = r[:, :, 0].reshape(b - a, F) @ w1[e].float().t() + r[:, :, 1].reshape(b - a, F) @ w2[e].float().t()
+        else:
+            ref = r @ w1[e].float().t()
+        assert float((outs[0][1][a:b].float() - ref).norm() / ref.norm()) <= 4e-3
