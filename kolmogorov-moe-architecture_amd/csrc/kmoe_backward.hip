@@ -148,8 +148,11 @@ __global__ __launch_bounds__(256) void silu_rows_kernel(const uint16_t* __restri
 //     dl[i_j] += w_j (dw_j - sum_l w_l dw_l)
 //   aux (scaled by the upstream gradient g of the aux loss):
 //     dl += g * (w_lb E / T * p (f - p.f) + w_z 2/T * lse * p),  f_e = counts[e] / (T k)
+// One thread per token, bound by latency: one wave a workgroup spreads 4096 tokens over 64 CUs
+// (four waves: 16 CUs, 9.7 -> 7.2 us at 16 experts, top-2).
+constexpr int DL_THREADS = 64;
 template <int NE>
-__global__ __launch_bounds__(256) void router_dlogits_kernel(const float* __restrict__ logits, int64_t T, int E,
+__global__ __launch_bounds__(DL_THREADS) void router_dlogits_kernel(const float* __restrict__ logits, int64_t T, int E,
                                                              const int64_t* __restrict__ topk_idx,
                                                              const float* __restrict__ topk_w,
                                                              const float* __restrict__ dw, int k,
@@ -573,10 +576,10 @@ extern "C" int kmoe_router_dlogits(const float* logits, int64_t T, int E, const 
   KMOE_REQUIRE(E >= 1 && E <= KMOE_MAX_EXPERTS && k >= 0 && k <= E, KMOE_ERR_SHAPE, "kmoe_router_dlogits: E=%d k=%d",
                E, k);
   if (T == 0) return KMOE_OK;
-  const dim3 grid((unsigned)kmoe::ceil_div<int64_t>(T, 256));
+  const dim3 grid((unsigned)kmoe::ceil_div<int64_t>(T, DL_THREADS));
   hipStream_t s = kmoe::as_stream(stream);
 #define KMOE_DL(NE_) \
-  hipLaunchKernelGGL(router_dlogits_kernel<NE_>, grid, dim3(256), 0, s, logits, T, E, topk_idx, topk_w, dw, k, counts, \
+  hipLaunchKernelGGL(router_dlogits_kernel<NE_>, grid, dim3(DL_THREADS), 0, s, logits, T, E, topk_idx, topk_w, dw, k, counts, \
                      grad_aux, w_lb, w_z, dlogits)
   if (E <= 8)
     KMOE_DL(8);
