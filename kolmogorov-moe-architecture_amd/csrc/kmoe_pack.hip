@@ -163,22 +163,28 @@ __global__ __launch_bounds__(256) void pack_t16_kernel(const void* __restrict__ 
 }
 
 // Zeroes what pack_t16_kernel leaves: in every packed row the elements [valid_cols,
-// out_ld), and the whole rows that no input column maps to.  One thread per row; the
-// pad of a row that holds data starts at an 8-byte boundary (valid_cols % 4 == 0) or
-// is first finished element by element.
+// out_ld), and the whole rows that no input column maps to.  PAD_LANES neighbouring threads
+// per row store 8 bytes each side by side (one thread per row stored a 128-byte pad as 16
+// single stores, each instruction touching 64 rows); a pad that does not start at an 8-byte
+// boundary (valid_cols % 4 != 0) is first finished element by element.  d 2048, F 2816, 16
+// experts, w13 and w3 together: 16.9 -> 11.4 us.
+constexpr int PAD_LANES = 16;
+inline dim3 pad_grid(int64_t n_rows) { return dim3((unsigned)kmoe::ceil_div<int64_t>(n_rows * PAD_LANES, 256)); }
 __global__ __launch_bounds__(256) void pack_pad_kernel(uint16_t* __restrict__ out, int64_t n_rows, int out_ld,
                                                        int valid_cols, int rows_per_expert, int valid_in_cols,
                                                        bool gate_up) {
-  const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t row = (int64_t)blockIdx.x * (256 / PAD_LANES) + threadIdx.x / PAD_LANES;
   if (row >= n_rows) return;
+  const int lane = threadIdx.x % PAD_LANES;
   const int pr = (int)(row % rows_per_expert);
   // the input column this packed row holds (gate_up: w1 / w2 column f of block f/128)
   const int c = gate_up ? (pr / 256) * 128 + (pr % 128) : pr;
   uint16_t* p = out + row * out_ld;
-  int from = c >= valid_in_cols ? 0 : valid_cols;
-  for (; (from & 3) != 0 && from < out_ld; ++from) p[from] = 0;
+  const int from = c >= valid_in_cols ? 0 : valid_cols;
+  const int whole = (from + 3) & ~3;
+  if (from + lane < min(whole, out_ld)) p[from + lane] = 0;
   uint64_t* w = reinterpret_cast<uint64_t*>(p);
-  for (int i = from / 4; i < out_ld / 4; ++i) w[i] = 0ull;
+  for (int i = whole / 4 + lane; i < out_ld / 4; i += PAD_LANES) w[i] = 0ull;
 }
 
 // Backward packed layouts (rows K-contiguous, WPAD bytes after every row, zero padded):
@@ -375,9 +381,9 @@ extern "C" int kmoe_pack_weights(const void* w1, const void* w2, const void* w3,
     else
       KMOE_PACK16(false);
 #undef KMOE_PACK16
-    hipLaunchKernelGGL(pack_pad_kernel, dim3((unsigned)kmoe::ceil_div<int64_t>(E * rows13, 256)), dim3(256), 0, s, o13,
+    hipLaunchKernelGGL(pack_pad_kernel, pad_grid((int64_t)E * rows13), dim3(256), 0, s, o13,
                        (int64_t)E * rows13, ld13, d, (int)rows13, F, true);
-    hipLaunchKernelGGL(pack_pad_kernel, dim3((unsigned)kmoe::ceil_div<int64_t>(E * rows3, 256)), dim3(256), 0, s, o3,
+    hipLaunchKernelGGL(pack_pad_kernel, pad_grid((int64_t)E * rows3), dim3(256), 0, s, o3,
                        (int64_t)E * rows3, ld3, F, (int)rows3, d, false);
     return kmoe::check_launch("kmoe_pack_weights");
   }
@@ -536,9 +542,9 @@ extern "C" int kmoe_pack_weights_plain(const void* w1, const void* w2, int w_dty
     hipLaunchKernelGGL(pack_t16_kernel<false>, g1, dim3(256), 0, s, w1, d, F, (int64_t)d * F, 0, false, o1, r1, ld1);
     hipLaunchKernelGGL(pack_t16_kernel<false>, g2, dim3(256), 0, s, w2, F, d, (int64_t)d * F, 0, false, o2, r2, ld2);
   }
-  hipLaunchKernelGGL(pack_pad_kernel, dim3((unsigned)kmoe::ceil_div<int64_t>(E * r1, 256)), dim3(256), 0, s, o1,
+  hipLaunchKernelGGL(pack_pad_kernel, pad_grid((int64_t)E * r1), dim3(256), 0, s, o1,
                      (int64_t)E * r1, ld1, d, (int)r1, F, false);
-  hipLaunchKernelGGL(pack_pad_kernel, dim3((unsigned)kmoe::ceil_div<int64_t>(E * r2, 256)), dim3(256), 0, s, o2,
+  hipLaunchKernelGGL(pack_pad_kernel, pad_grid((int64_t)E * r2), dim3(256), 0, s, o2,
                      (int64_t)E * r2, ld2, F, (int)r2, d, false);
   return kmoe::check_launch("kmoe_pack_weights_plain");
 }

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from kmoe import AdvancedMoEConfig, MoELayer, checkpoint as C
+from kmoe import AdvancedMoEConfig, MoELayer, _lib, checkpoint as C
 
 pytestmark = pytest.mark.gpu
 
@@ -141,3 +141,27 @@ def test_bf16_packs_match_host_layout(dev, E, d, F, wdtype):
             w13t[e, i, c[ok & (half == 1)]] = b2[e, i, src_f[ok & (half == 1)]]
     assert np.array_equal(bw.w3n.cpu().view(torch.int16).numpy().reshape(w3n.shape), w3n)
     assert np.array_equal(bw.w13t.cpu().view(torch.int16).numpy().reshape(w13t.shape), w13t)
+
+
+@pytest.mark.parametrize("E,d,F", [(1, 64, 1), (2, 128, 13), (3, 192, 126), (2, 320, 131), (2, 256, 256)])
+def test_bf16_packs_zero_their_padding(dev, E, d, F):
+    """Into buffers full of ones bits: the pad after each packed row (at any F % 4) and the
+    rows that hold no weight are zero, and with all weights 1.0 every other element is 1.0."""
+    lib = _lib.load()
+    w1 = torch.ones(E, d, F, dtype=torch.bfloat16, device=dev)
+    w3 = torch.ones(E, F, d, dtype=torch.bfloat16, device=dev)
+    Fp, dp = (F + 127) // 128 * 128, (d + 255) // 256 * 256
+    o13 = torch.full((E, Fp // 128, 2, 128, d + 64), -1, dtype=torch.int16, device=dev)
+    o3 = torch.full((E, dp, Fp + 64), -1, dtype=torch.int16, device=dev)
+    assert o13.numel() * 2 == lib.kmoe_packed_w13_bytes(E, d, F, _lib.DTYPE_BF16)
+    assert o3.numel() * 2 == lib.kmoe_packed_w3_bytes(E, d, F, _lib.DTYPE_BF16)
+    _lib.call("kmoe_pack_weights", _lib.ptr(w1), _lib.ptr(w1), _lib.ptr(w3), _lib.DTYPE_BF16, E, d, F, _lib.DTYPE_BF16,
+              _lib.ptr(o13), None, _lib.ptr(o3), None, _lib.stream_ptr(dev))
+    torch.cuda.synchronize()
+    one = int(torch.ones(1, dtype=torch.bfloat16).view(torch.int16))
+    want13 = torch.zeros(E, Fp, d + 64, dtype=torch.int16)
+    want13[:, :F, :d] = one
+    want13 = want13.view(E, Fp // 128, 1, 128, d + 64).expand(-1, -1, 2, -1, -1)
+    want3 = torch.zeros(E, dp, Fp + 64, dtype=torch.int16)
+    want3[:, :d, :F] = one
+    assert torch.equal(o13.cpu(), want13) and torch.equal(o3.cpu(), want3)
