@@ -1,5 +1,7 @@
 // Grouped expert products: launch choice and C entry points.  The kernels are in
 // kmoe_gemm_tile.h.
+#include <algorithm>
+
 #include "kmoe_gemm_tile.h"
 
 using namespace kmoe_tiles;
@@ -72,8 +74,8 @@ int launch_gemm(bool gate_up, bool fp8, const void* A, const float* a_scale, con
   g.gu_out = static_cast<uint16_t*>(gu_out);
   g.Cf = nullptr;
   // tile loads address a 2 GiB buffer window from the tile's first A / B row (from
-  // the first row of A when gathering)
-  if ((int64_t)(BM + 1) * g.ldb_bytes >= ((int64_t)1 << 31) ||
+  // the first row of A when gathering); with B2 a row of A is twice one of B
+  if ((int64_t)(BM + 1) * std::max(g.lda_bytes, g.ldb_bytes) >= ((int64_t)1 << 31) ||
       (row_token && (n_a_rows + 1) * g.lda_bytes >= ((int64_t)1 << 31))) {
     kmoe::set_error("kmoe gemm: operand too large for 32-bit tile offsets (K bytes %d)", kbytes);
     return KMOE_ERR_SHAPE;

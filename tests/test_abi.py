@@ -106,6 +106,16 @@ def test_gemm_and_combine_validation(lib):
                 FAKE, _lib.DTYPE_BF16, NULL)[0] == -2
 
 
+def test_grouped_weights_operand_window(lib):
+    """With two weight matrices a row of A is K elements and one of b or b2 half of that: the
+    256-row tile's A rows must fit the 2 GiB load window too (at K = 2^22 + 512 those of b
+    do and those of A end at 2 GiB + 128 KiB)"""
+    K = (1 << 22) + 512
+    assert 257 * K < 1 << 31 <= 256 * 2 * K
+    rc, msg = _err(lib, "kmoe_gemm_grouped_weights", FAKE, FAKE, 1, K, 256, FAKE, FAKE, 256, FAKE, 256, NULL)
+    assert rc == -2 and "too large" in msg
+
+
 def test_select_validation(lib):
     assert _err(lib, "kmoe_ec_select", FAKE, 1, 100, 4, 101, 1, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, NULL, 0,
                 NULL)[0] == -2
