@@ -41,15 +41,7 @@ int launch_gemm(bool gate_up, bool fp8, const void* A, const float* a_scale, con
                 const void* B2 = nullptr) {
   const int eb = fp8 ? 1 : 2;
   const int64_t slots = kmoe::ceil_div<int64_t>(max_rows, BM) + E;
-  // every tile of the worst-case slot count, plus one narrow tile per resident
-  // workgroup for the split tail (e4m3: one workgroup per CU and the
-  // narrow tiles, or with a single K-step every tile in halves)
   const int n_cu = kmoe::cu_count();
-  const int64_t blocks = !fp8 ? slots * n_tiles + n_cu : K >= 2 * KB ? 2 * n_cu : 2 * slots * n_tiles;
-  if (blocks > 0x7fffffff) {
-    kmoe::set_error("kmoe gemm: grid too large");
-    return KMOE_ERR_SHAPE;
-  }
   const int kbytes = K * eb;
   if (kbytes % KB != 0) {
     kmoe::set_error("kmoe gemm: K bytes %d not a multiple of %d", kbytes, KB);
@@ -73,6 +65,14 @@ int launch_gemm(bool gate_up, bool fp8, const void* A, const float* a_scale, con
   g.C2 = static_cast<uint16_t*>(C2);
   g.gu_out = static_cast<uint16_t*>(gu_out);
   g.Cf = nullptr;
+  // every tile of the worst-case slot count, plus one narrow tile per resident
+  // workgroup for the split tail (e4m3 in the full-tile loop: one workgroup per CU and the
+  // narrow tiles, else every tile in halves)
+  const int64_t blocks = !fp8 ? slots * n_tiles + n_cu : full_tile_loop(g) ? 2 * n_cu : 2 * slots * n_tiles;
+  if (blocks > 0x7fffffff) {
+    kmoe::set_error("kmoe gemm: grid too large");
+    return KMOE_ERR_SHAPE;
+  }
   // tile loads address a 2 GiB buffer window from the tile's first A / B row (from
   // the first row of A when gathering); with B2 a row of A is twice one of B
   if ((int64_t)(BM + 1) * std::max(g.lda_bytes, g.ldb_bytes) >= ((int64_t)1 << 31) ||

@@ -309,6 +309,14 @@ struct GemmArgs {
   float* Cf;
 };
 
+// Whether the full tiles of an e4m3 product run in gemm_full_tiles: its pipeline holds two
+// K-steps, and its epilogue's buffer stores reach 2 GiB from the tile's first row of C (and of
+// gu_out, whose rows are twice as long).  Otherwise every tile runs as two narrow
+// ones, whose stores take 64-bit addresses.
+__host__ __device__ inline bool full_tile_loop(const GemmArgs& g) {
+  return g.k_bytes >= 2 * KB && BM * g.ldc * (g.gu_out ? 4 : 2) < (int64_t)1 << 31;
+}
+
 // Stores a tile staged in LDS (BM rows of OCPR 16-byte chunks, row stride OSTR bytes)
 // to the rows [m0, m_end) of `out` (row stride ld elements, chunk ch at out + 8 ch;
 // chunks from column col0 + 8 ch >= n_valid are not stored).  A thread always handles
@@ -891,7 +899,7 @@ static_assert(FT_LDS <= GEMM_LDS, "LDS of the full-tile loop");
 // e4m3 tile has half the K-steps of a bf16 one: the layer of 8192 tokens (6144 kept), d
 // 2048, F 2816 375 -> 358 us against one workgroup per tile.  (bf16 tiles the same way: 1045
 // -> 1025 us at 16384 tokens, eleven rounds, but 2% slower at one to three rounds; they
-// stay one workgroup per tile.)  Needs at least two K-steps.
+// stay one workgroup per tile.)  For products with full_tile_loop().
 // NMA (4, 2 or 0, per tile and wave): the wave's 32-row blocks that hold rows of the
 // expert; the others' fragment reads, MFMAs and stores are skipped.  The waves of a
 // workgroup may differ in NMA: loads, LDS writes and barriers are the same.
@@ -1225,9 +1233,9 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
 // of 1/split of its columns (the full K), which all run at once.  A narrow tile
 // computes every output element with the same MFMA sequence as the full tile, so
 // the results are identical.  split = 1 keeps the tail tiles whole.
-// e4m3 products of at least two K-steps: the full rounds (and whole tail tiles) go to
-// gemm_full_tiles on the first n_cu workgroups, the narrow tiles to the ones after them (a
-// single K-step: all tiles in halves).
+// e4m3 products with full_tile_loop(): the full rounds (and whole tail tiles) go to
+// gemm_full_tiles on the first n_cu workgroups, the narrow tiles to the ones after them
+// (without it: all tiles in halves).
 template <bool GATE_UP, bool FP8, bool GATHER, bool SAVE_GU = false, bool RSCALE = false, bool DUAL = false>
 __global__ __launch_bounds__(GEMM_THREADS, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void grouped_gemm_kernel(
     GemmArgs g, const int32_t* __restrict__ offsets, int E, int n_tiles, int n_cu) {
@@ -1245,14 +1253,14 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) __attribute__((amdgpu_waves_per_eu
   }
   const int L = blockIdx.x;
   if constexpr (FP8) {
-    const bool one_step = g.k_bytes < 2 * KB;
-    if (one_step)
+    const bool halves = !full_tile_loop(g);
+    if (halves)
       split = 2;
     else if (L < n_cu) {
       gemm_full_tiles<GATE_UP, SAVE_GU>(g, lds, st, E, n_tiles, n_cu, base, split == 1 ? n_all : base);
       return;
     }
-    const int first = one_step ? 0 : base, u = one_step ? L : L - n_cu;
+    const int first = halves ? 0 : base, u = halves ? L : L - n_cu;
     if (split == 1 || u >= (n_all - first) * split) return;
     int slot, nt, e, m0, m_end;
     dense_tile(first + u / split, st.n_slots, n_tiles, slot, nt);

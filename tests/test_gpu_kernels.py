@@ -759,6 +759,36 @@ def test_full_tile_loop(dev, path, d):
             assert rel(gu[s:t], packed) <= 4e-3, (path, d, e, counts[e])
 
 
+def test_fp8_outputs_past_2gib(dev):
+    """e4m3 gate/up whose 256 rows of saved pre-activations end past 2 GiB: the last rows and
+    columns of h and gu against fp32 products of the decoded operands (bar 4e-3 rel-L2: one
+    bf16 rounding); a store window that ends before them leaves the zeros they start with."""
+    from kmoe import _lib
+
+    d, F, A = 256, (1 << 21) + 128, 256
+    assert A * 4 * F > 1 << 31
+    g = torch.Generator(device=dev).manual_seed(5)
+    # codes of +-2^-6 .. +-15 and no NaN; rows of w13: 128 gate, 128 up, each padded by 128 bytes
+    code = lambda *s: torch.randint(8, 0x60, s, generator=g, device=dev, dtype=torch.uint8) | (
+        torch.randint(0, 2, s, generator=g, device=dev, dtype=torch.uint8) << 7)
+    xq, xs = code(A, d), torch.rand(A, generator=g, device=dev) * 1e-2
+    w13, ws = torch.zeros(2 * F, d + 128, device=dev, dtype=torch.uint8), torch.rand(2 * F, generator=g, device=dev) * 1e-2
+    w13[:, :d] = code(2 * F, d)
+    off = torch.tensor([0, A], dtype=torch.int32, device=dev)
+    h = torch.zeros(A, F, device=dev, dtype=torch.bfloat16)
+    gu = torch.zeros(A, 2 * F, device=dev, dtype=torch.bfloat16)
+    p = _lib.ptr
+    _lib.call("kmoe_gemm_gate_up_fp8_gu", p(xq), p(xs), p(off), 1, d, F, A, p(w13), p(ws), p(h), p(gu), ops._stream(h))
+    val = lambda q, s: q.view(torch.float8_e4m3fn).float() * s[:, None]
+    for r in (0, 192, 254):
+        for c in (0, F - 128):
+            ref = val(xq[r:r + 2], xs[r:r + 2]) @ val(w13[2 * c:2 * c + 256, :d], ws[2 * c:2 * c + 256]).t()
+            got = gu[r:r + 2, 2 * c:2 * c + 256].float()
+            assert float((got - ref).norm() / ref.norm()) <= 4e-3, (r, c)
+            hr = torch.nn.functional.silu(ref[:, :128]) * ref[:, 128:]
+            assert float((h[r:r + 2, c:c + 128].float() - hr).norm() / hr.norm()) <= 4e-3, (r, c)
+
+
 # ------------------------------------------------------------------ few rows per expert
 @pytest.mark.parametrize("d,F,counts", [(64, 40, [1, 0, 2]), (128, 128, [16, 17, 1, 0]), (320, 130, [32, 33, 15, 31]),
                                         (2048, 704, [1] + [0] * 6 + [3, 10, 64]), (192, 2816, [2, 1])])
