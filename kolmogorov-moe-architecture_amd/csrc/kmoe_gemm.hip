@@ -66,13 +66,15 @@ int launch_gemm(bool gate_up, bool fp8, const void* A, const float* a_scale, con
   g.gu_out = static_cast<uint16_t*>(gu_out);
   g.Cf = nullptr;
   // every tile of the worst-case slot count, plus one narrow tile per resident
-  // workgroup for the split tail (e4m3 in the full-tile loop: one workgroup per CU and the
-  // narrow tiles, else every tile in halves)
-  const int64_t blocks = !fp8 ? slots * n_tiles + n_cu : full_tile_loop(g) ? 2 * n_cu : 2 * slots * n_tiles;
+  // workgroup for the split tail
+  int64_t blocks = slots * n_tiles + n_cu;
   if (blocks > 0x7fffffff) {
     kmoe::set_error("kmoe gemm: grid too large");
     return KMOE_ERR_SHAPE;
   }
+  // e4m3: one workgroup per CU for the full-tile loop and one for the narrow tiles after it;
+  // without the loop every tile in halves, or in quarters on at most n_cu workgroups
+  if (fp8) blocks = full_tile_loop(g) ? 2 * n_cu : std::max<int64_t>(2 * slots * n_tiles, n_cu);
   // tile loads address a 2 GiB buffer window from the tile's first A / B row (from
   // the first row of A when gathering); with B2 a row of A is twice one of B
   if ((int64_t)(BM + 1) * std::max(g.lda_bytes, g.ldb_bytes) >= ((int64_t)1 << 31) ||

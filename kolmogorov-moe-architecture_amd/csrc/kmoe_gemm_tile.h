@@ -311,8 +311,8 @@ struct GemmArgs {
 
 // Whether the full tiles of an e4m3 product run in gemm_full_tiles: its pipeline holds two
 // K-steps, and its epilogue's buffer stores reach 2 GiB from the tile's first row of C (and of
-// gu_out, whose rows are twice as long).  Otherwise every tile runs as two narrow
-// ones, whose stores take 64-bit addresses.
+// gu_out, whose rows are twice as long).  Otherwise every tile runs as narrow ones,
+// whose stores take 64-bit addresses.
 __host__ __device__ inline bool full_tile_loop(const GemmArgs& g) {
   return g.k_bytes >= 2 * KB && BM * g.ldc * (g.gu_out ? 4 : 2) < (int64_t)1 << 31;
 }
@@ -900,7 +900,7 @@ static_assert(FT_LDS <= GEMM_LDS, "LDS of the full-tile loop");
 // 2048, F 2816 375 -> 358 us against one workgroup per tile.  (bf16 tiles the same way: 1045
 // -> 1025 us at 16384 tokens, eleven rounds, but 2% slower at one to three rounds; they
 // stay one workgroup per tile.)  For products with full_tile_loop().
-// NMA (4, 2 or 0, per tile and wave): the wave's 32-row blocks that hold rows of the
+// NMA (4, 2, 1 or 0, per tile and wave): the wave's 32-row blocks that hold rows of the
 // expert; the others' fragment reads, MFMAs and stores are skipped.  The waves of a
 // workgroup may differ in NMA: loads, LDS writes and barriers are the same.
 // a_scale per A row, b_scale per B row (global row index).
@@ -1211,12 +1211,14 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
       __builtin_amdgcn_sched_barrier(0);
       epilogue(cur, set, nma_tag);
     };
-    // row blocks of this wave holding rows (wave-uniform): 4 (more than 64 rows), 2, 0
+    // row blocks of this wave holding rows (wave-uniform): 4 (more than 64 rows), 2, 1, 0
     const int wrows = cur.m_end - cur.m0 - wm * 128;
     if (wrows > 64)
       body(std::integral_constant<int, 4>{});
-    else if (wrows > 0)
+    else if (wrows > 32)
       body(std::integral_constant<int, 2>{});
+    else if (wrows > 0)
+      body(std::integral_constant<int, 1>{});
     else
       body(std::integral_constant<int, 0>{});
     cur = nx;
@@ -1235,7 +1237,7 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
 // the results are identical.  split = 1 keeps the tail tiles whole.
 // e4m3 products with full_tile_loop(): the full rounds (and whole tail tiles) go to
 // gemm_full_tiles on the first n_cu workgroups, the narrow tiles to the ones after them
-// (without it: all tiles in halves).
+// (without it: all tiles in halves or quarters).
 template <bool GATE_UP, bool FP8, bool GATHER, bool SAVE_GU = false, bool RSCALE = false, bool DUAL = false>
 __global__ __launch_bounds__(GEMM_THREADS, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void grouped_gemm_kernel(
     GemmArgs g, const int32_t* __restrict__ offsets, int E, int n_tiles, int n_cu) {
@@ -1253,14 +1255,20 @@ __global__ __launch_bounds__(GEMM_THREADS, 1) __attribute__((amdgpu_waves_per_eu
   }
   const int L = blockIdx.x;
   if constexpr (FP8) {
+    // without the loop every tile is narrow, in quarters where all of them then fit at once
     const bool halves = !full_tile_loop(g);
-    if (halves)
-      split = 2;
-    else if (L < n_cu) {
+    if (halves) split = 4 * n_all <= n_cu ? 4 : 2;
+    // the narrow tiles wait behind n_cu workgroups only where those have tiles of their own
+    // (4 experts, d 256, F 352, 1024 rows: gate/up + down 13.8 us behind 256 workgroups
+    // without one, 12.8 from the first on), and a single K-step takes quarters where all fit
+    // at once (16 experts, d 128, F 256, 128 rows: 14.5 us in halves, 12.1)
+    const int first = halves ? 0 : base;  // first narrow tile
+    const bool looped = !halves && (split == 1 || base > 0);
+    if (looped && L < n_cu) {
       gemm_full_tiles<GATE_UP, SAVE_GU>(g, lds, st, E, n_tiles, n_cu, base, split == 1 ? n_all : base);
       return;
     }
-    const int first = halves ? 0 : base, u = halves ? L : L - n_cu;
+    const int u = looped ? L - n_cu : L;
     if (split == 1 || u >= (n_all - first) * split) return;
     int slot, nt, e, m0, m_end;
     dense_tile(first + u / split, st.n_slots, n_tiles, slot, nt);

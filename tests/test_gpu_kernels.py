@@ -759,6 +759,42 @@ def test_full_tile_loop(dev, path, d):
             assert rel(gu[s:t], packed) <= 4e-3, (path, d, e, counts[e])
 
 
+@pytest.mark.parametrize("d", [128, 256, 384])
+@pytest.mark.parametrize("tiles_of_cus", [0.1, 0.25, 0.26, 0.5, 0.75, 1.1])
+def test_fp8_few_tiles(dev, d, tiles_of_cus):
+    """e4m3 products of fewer tiles than a round (from the first workgroup on: quarters up to
+    n_cu / 4 tiles, halves up to n_cu / 2, else whole, or a single K-step in quarters or
+    halves) and of little more, experts ending in slots of 1 to 161 rows (0 to 4 row blocks of
+    a wave): gate/up and down against fp32 products of the decoded operands (bar 4e-3 rel-L2:
+    one bf16 rounding)."""
+    n_cu = torch.cuda.get_device_properties(dev).multi_processor_count
+    F = 256  # two column tiles a slot (down: d / 256)
+    last = [1, 31, 32, 33, 64, 65, 128, 129, 160, 161]
+    n_slots = max(int(n_cu * tiles_of_cus / 2), len(last))
+    each = [n_slots // len(last) + (i < n_slots % len(last)) for i in range(len(last))]
+    counts = [256 * (n - 1) + r for n, r in zip(each, last)]
+    E, A = len(counts), sum(counts)
+    off_l = np.concatenate([[0], np.cumsum(counts)])
+    off = torch.tensor(off_l, dtype=torch.int32, device=dev)
+    g = torch.Generator(device=dev).manual_seed(d)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    w1, w2, w3 = (bf16(rnd(*s) * s[1] ** -0.5) for s in ((E, d, F), (E, d, F), (E, F, d)))
+    pw = ops.pack_weights(w1, w2, w3, fp8=True)
+    w1, w2, w3 = (ops.fake_quant_cols_e4m3(w).float() for w in (w1, w2, w3))
+    xq, xs = ops.quant_rows_fp8(bf16(rnd(A, d)))
+    h = ops.gemm_gate_up(xq, xs, off, pw, A)
+    hq, hs = ops.quant_rows_fp8(h)
+    y = ops.gemm_down(hq, hs, off, pw, A)
+    val = lambda q, s: q.view(torch.float8_e4m3fn).float() * s[:, None]
+    rel = lambda a, b: float((a.float() - b).norm() / b.norm())
+    x, hv = val(xq, xs), val(hq, hs)
+    for e in range(E):
+        s, t = int(off_l[e]), int(off_l[e + 1])
+        ref = torch.nn.functional.silu(x[s:t] @ w1[e]) * (x[s:t] @ w2[e])
+        assert rel(h[s:t, :F], ref) <= 4e-3, (e, counts[e])
+        assert rel(y[s:t], hv[s:t, :F] @ w3[e]) <= 4e-3, (e, counts[e])
+
+
 def test_fp8_outputs_past_2gib(dev):
     """e4m3 gate/up whose 256 rows of saved pre-activations end past 2 GiB: the last rows and
     columns of h and gu against fp32 products of the decoded operands (bar 4e-3 rel-L2: one
