@@ -874,6 +874,29 @@ def test_small_rows(dev, path, d, F, counts):
                 assert rel(gu[s:t, 2 * f + 128:2 * f + 128 + n], uu[:, f:f + n]) <= 4e-3
 
 
+@pytest.mark.parametrize("E,d,F,rows", [(64, 2048, 1408, 640), (64, 2048, 1408, 384), (16, 2048, 2816, 160)])
+def test_small_rows_leave_skewed_routing(dev, E, d, F, rows):
+    """Row counts at which one expert with all the rows would stream its weights for many
+    32-row slots run on the 256-row tiles: the same bits as under a larger bound on the rows
+    (which takes the tiles; the small-row kernel sums K in four parts)."""
+    g = torch.Generator(device=dev).manual_seed(rows)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    w1, w2, w3 = (bf16(rnd(*s) * s[1] ** -0.5) for s in ((E, d, F), (E, d, F), (E, F, d)))
+    pw = ops.pack_weights(w1, w2, w3)
+    A = 64 * E
+    x = bf16(rnd(A, d))
+    off = torch.full((E + 1,), rows, dtype=torch.int32, device=dev)
+    off[0] = 0
+    rt = torch.arange(A, dtype=torch.int32, device=dev)
+    h, hb = (ops.gemm_gate_up_rows(x, None, rt, off, pw, n)[:rows] for n in (rows, A))
+    assert torch.equal(h, hb)
+    hx = torch.zeros(A, h.shape[1], device=dev, dtype=torch.bfloat16)
+    hx[:rows] = h
+    y, yb = (ops.gemm_down(hx[:n], None, off, pw, n)[:rows] for n in (rows, A))
+    if rows // 32 * (d // 32) > 3 * torch.cuda.get_device_properties(dev).multi_processor_count or rows > 8 * E:
+        assert torch.equal(y, yb)
+
+
 # ------------------------------------------------------------------ weights read in place
 @pytest.mark.parametrize("d,F,counts", [(256, 256, [1, 0, 2]), (512, 768, [33, 0, 17, 5]), (512, 768, [1500, 17, 0, 2513]),
                                         (256, 1280, [257] * 40), (2048, 256, [600, 1])])
