@@ -7,6 +7,8 @@
 //   aux = w_lb * E * sum_e f_e P_e + w_z * mean_t lse_t^2      (moe.py:840-939)
 // with f_e = counts[e] / (T k) a constant (one-hot of the selections) and
 // P_e = mean_t p[t,e].
+#include <algorithm>
+
 #include "kmoe_common.h"
 
 namespace {
@@ -274,15 +276,24 @@ __global__ __launch_bounds__(ECD_THREADS) void ec_dlogits_kernel(const float* __
   }
 }
 
-// Router MLP backward over a block of RB_TOK tokens (256 threads, RB_TPT per token):
+// Router MLP backward, RB_TOK tokens at a time (256 threads, RB_TPT per token):
 //   s = silu(a), ds = dl w_out, da = ds * silu'(a)      -> da (T, 128) bf16
-//   partial[b][e][j] = sum_{t in block} dl[t,e] s[t,j]  -> reduced by router_reduce_kernel
+//   partial[b][e][j] = sum_{t of block b} dl[t,e] s[t,j] -> reduced by reduce_partials_kernel
 // a (T, 128) f32 is the saved pre-activation of the d -> 128 layer.
-// 16 tokens a block: with 64 the 64 blocks of 4096 tokens left three CUs in four idle, each
-// walking 64 tokens serially for dW_out (4096 tokens, 16 experts: 24.0 -> 11.2 us).
+// Bound by latency while the tokens are few: 16 at a time give 4096 tokens 256 workgroups (of
+// 64 tokens: 64, each walking them serially for dW_out; 16 experts 21.1 -> 10.1 us).  At most
+// three workgroups per CU, each summing several groups of tokens in registers: more partial
+// sums cost more than they hide (64 tokens a workgroup / one group a workgroup / at most three
+// per CU, us: 16384 tokens, 64 experts 50.4 / 50.7 / 45.5; 65536 tokens, 4 experts 32.9 / 41.6
+// / 31.0, 16 experts 53.7 / 56.0 / 37.8; at most two or four per CU are slower at one end).
 constexpr int RB_TOK = 16;
 constexpr int RB_TPT = 256 / RB_TOK;
+constexpr int RB_WGS_PER_CU = 3;
 constexpr int RH = KMOE_ROUTER_HIDDEN;
+// Workgroups of the launch: rows of the workspace.
+int64_t router_bwd_blocks(int64_t T) {
+  return std::min<int64_t>(kmoe::ceil_div<int64_t>(T, RB_TOK), (int64_t)RB_WGS_PER_CU * kmoe::cu_count());
+}
 template <int NE>
 __global__ __launch_bounds__(256) void router_mlp_bwd_kernel(const float* __restrict__ dl,
                                                              const float* __restrict__ a, int64_t T, int E,
@@ -293,33 +304,43 @@ __global__ __launch_bounds__(256) void router_mlp_bwd_kernel(const float* __rest
   __shared__ float s_l[RB_TOK][RH + 1];
   __shared__ float dl_l[RB_TOK][NE];
   const int tid = threadIdx.x;
-  const int64_t t0 = (int64_t)blockIdx.x * RB_TOK;
   for (int i = tid; i < NE * RH; i += 256) wo[i / RH][i % RH] = i / RH < E ? bf16_to_f32(w_out[i]) : 0.0f;
-  for (int i = tid; i < RB_TOK * NE; i += 256) {
-    const int tl = i / NE, e = i % NE;
-    dl_l[tl][e] = (t0 + tl < T && e < E) ? dl[(t0 + tl) * E + e] : 0.0f;
-  }
-  __syncthreads();
   const int tl = tid / RB_TPT, part = tid % RB_TPT;
-  const int64_t t = t0 + tl;
-  for (int jj = 0; jj < RH / RB_TPT; ++jj) {
-    const int j = part + RB_TPT * jj;
-    const float av = t < T ? a[t * RH + j] : 0.0f;
-    const float sg = 1.0f / (1.0f + __expf(-av));
-    const float s = av * sg;
-    float ds = 0.0f;
+  // dW_out of the block's tokens: thread holds the (e, j) pairs tid, tid + 256, ...
+  constexpr int NP = NE * RH / 256;
+  float acc[NP];
 #pragma unroll
-    for (int e = 0; e < NE; ++e) ds = fmaf(dl_l[tl][e], wo[e][j], ds);
-    s_l[tl][j] = t < T ? s : 0.0f;
-    if (t < T) da[t * RH + j] = f32_to_bf16(ds * sg * (1.0f + av * (1.0f - sg)));
+  for (int p = 0; p < NP; ++p) acc[p] = 0.0f;
+  for (int64_t t0 = (int64_t)blockIdx.x * RB_TOK; t0 < T; t0 += (int64_t)gridDim.x * RB_TOK) {
+    __syncthreads();  // the previous tokens' sums have read s_l and dl_l
+    for (int i = tid; i < RB_TOK * NE; i += 256) {
+      const int q = i / NE, e = i % NE;
+      dl_l[q][e] = (t0 + q < T && e < E) ? dl[(t0 + q) * E + e] : 0.0f;
+    }
+    __syncthreads();
+    const int64_t t = t0 + tl;
+    for (int jj = 0; jj < RH / RB_TPT; ++jj) {
+      const int j = part + RB_TPT * jj;
+      const float av = t < T ? a[t * RH + j] : 0.0f;
+      const float sg = 1.0f / (1.0f + __expf(-av));
+      const float s = av * sg;
+      float ds = 0.0f;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) ds = fmaf(dl_l[tl][e], wo[e][j], ds);
+      s_l[tl][j] = t < T ? s : 0.0f;
+      if (t < T) da[t * RH + j] = f32_to_bf16(ds * sg * (1.0f + av * (1.0f - sg)));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const int i = tid + 256 * p, e = i / RH, j = i % RH;
+      for (int q = 0; q < RB_TOK; ++q) acc[p] = fmaf(dl_l[q][e], s_l[q][j], acc[p]);
+    }
   }
-  __syncthreads();
-  // partial dW_out of the block: thread handles (e, j) pairs tid, tid + 256, ...
-  for (int i = tid; i < NE * RH; i += 256) {
-    const int e = i / RH, j = i % RH;
-    float acc = 0.0f;
-    for (int q = 0; q < RB_TOK; ++q) acc = fmaf(dl_l[q][e], s_l[q][j], acc);
-    if (e < E) partial[(int64_t)blockIdx.x * E * RH + e * RH + j] = acc;
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const int i = tid + 256 * p;
+    if (i / RH < E) partial[(int64_t)blockIdx.x * E * RH + i] = acc[p];
   }
 }
 
@@ -604,7 +625,7 @@ extern "C" int kmoe_ec_dlogits(const float* logits, int B, int S, int E, const i
 }
 
 extern "C" size_t kmoe_router_bwd_workspace_bytes(int64_t T, int E) {
-  return (size_t)kmoe::ceil_div<int64_t>(T, RB_TOK) * (size_t)E * RH * sizeof(float);
+  return (size_t)router_bwd_blocks(T) * (size_t)E * RH * sizeof(float);
 }
 
 extern "C" int kmoe_router_mlp_bwd(const float* dlogits, const float* hidden_pre, int64_t T, int E, const void* w_out,
@@ -618,7 +639,7 @@ extern "C" int kmoe_router_mlp_bwd(const float* dlogits, const float* hidden_pre
   KMOE_REQUIRE(workspace_bytes >= kmoe_router_bwd_workspace_bytes(T, E), KMOE_ERR_WORKSPACE,
                "kmoe_router_mlp_bwd: workspace %zu < %zu", workspace_bytes, kmoe_router_bwd_workspace_bytes(T, E));
   if (T == 0) return KMOE_OK;
-  const int64_t nblk = kmoe::ceil_div<int64_t>(T, RB_TOK);
+  const int64_t nblk = router_bwd_blocks(T);
   hipStream_t s = kmoe::as_stream(stream);
   float* part = static_cast<float*>(workspace);
 #define KMOE_MB(NE_)                                                                                        \

@@ -116,6 +116,14 @@ def test_grouped_weights_operand_window(lib):
     assert rc == -2 and "too large" in msg
 
 
+def test_router_bwd_workspace_is_bounded(lib):
+    """The partial sums of the router's backward: one row of E x 128 floats per 16 tokens, at
+    most three rows per CU however many tokens"""
+    f = lib.kmoe_router_bwd_workspace_bytes
+    assert f(0, 4) == 0 and f(1, 4) == 4 * 128 * 4 and f(4096, 16) == 256 * 16 * 128 * 4
+    assert f(1 << 16, 4) == f(1 << 20, 4) <= (1 << 16) // 64 * 4 * 128 * 4
+
+
 def test_select_validation(lib):
     assert _err(lib, "kmoe_ec_select", FAKE, 1, 100, 4, 101, 1, FAKE, FAKE, FAKE, FAKE, FAKE, FAKE, NULL, 0,
                 NULL)[0] == -2

@@ -322,3 +322,32 @@ def test_backward_balanced_routing(dev):
     plain = torch.topk(r.logits, k, dim=1).indices.cpu()
     assert (plain.sort(1).values != idx.sort(1).values).any(), "the capacity rule must have moved some picks"
     _check(errs)
+
+
+@pytest.mark.parametrize("E,T", [(3, 1), (5, 17), (16, 4096), (64, 12287), (8, 12289), (64, 30001), (4, 70003)])
+def test_router_mlp_bwd(dev, E, T):
+    """da and dW_out of the router MLP against fp64 of the same f32 operands, from one token to
+    several groups of 16 tokens a workgroup (above 12288 tokens on 256 CUs), ragged ends.  Bars:
+    one bf16 rounding of da (2^-9 at most per value); dW_out is an f32 sum in chains of at most
+    a few hundred terms (1e-5), and the same bits again."""
+    from kmoe import _lib, ops
+
+    g = torch.Generator(device=dev).manual_seed(T)
+    dl, a = (torch.randn(T, n, generator=g, device=dev) for n in (E, 128))
+    w = torch.randn(E, 128, generator=g, device=dev).to(torch.bfloat16)
+    nb = _lib.load().kmoe_router_bwd_workspace_bytes(T, E)
+    p = _lib.ptr
+    outs = []
+    for _ in range(2):
+        ws = torch.full((nb // 4,), float("nan"), device=dev)
+        da = torch.full((T, 128), float("nan"), device=dev, dtype=torch.bfloat16)
+        dw = torch.full((E, 128), float("nan"), device=dev)
+        _lib.call("kmoe_router_mlp_bwd", p(dl), p(a), T, E, p(w), p(da), p(dw), _lib.DTYPE_F32, p(ws), nb,
+                  ops._stream(da))
+        outs.append((da, dw))
+    a64 = a.double().cpu().requires_grad_(True)
+    s = torch.nn.functional.silu(a64)
+    (s @ w.double().cpu().t()).backward(dl.double().cpu())
+    assert _rel(outs[0][0], a64.grad) <= 4e-3
+    assert _rel(outs[0][1], dl.double().cpu().t() @ s.detach()) <= 1e-5
+    assert all(torch.equal(x, y) for x, y in zip(*outs))
