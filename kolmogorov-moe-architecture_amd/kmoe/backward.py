@@ -18,6 +18,7 @@ Data flow (A = routed rows, grouped by expert):
 """
 from __future__ import annotations
 
+import math
 from typing import NamedTuple, Optional
 
 import torch
@@ -26,13 +27,23 @@ from . import _lib, ops
 from ._lib import ptr
 
 _BF16 = torch.bfloat16
-# token rows per split-K segment of the router's weight gradient (128 x d outputs are few
-# tiles: at 4096 tokens, d 2048, segments of 512 rows made 64 workgroups, of 128 rows 256)
-WG_SPLIT = 128
 
 
 def _ru(a: int, b: int) -> int:
     return (a + b - 1) // b * b
+
+
+def router_wgrad_rows(T: int, d: int, n_cu: int) -> int:
+    """Token rows per split-K segment of the router's weight gradient dW_in (128, d): a
+    multiple of the 64-row K-step, at most MAX_EXPERTS segments.  A workgroup walks one
+    segment's rows serially for 256 of the d columns, and every segment adds a 128 x d f32
+    partial sum to write and to reduce.  Best measured: one round of workgroups on the CUs, and
+    fewer, longer segments at few tokens, sqrt(T d / 200) rows (us with segments of 128 / 256 /
+    512 rows: 4096 tokens, d 256 14.8 / 16.2 / 21.4 (64 here), d 2048 30.1 / 27.3 / 31.2 (192);
+    8192 tokens, d 2048 39.5 / 30.2 / 32.4 (256), d 8192 164 / 104 / 78 (1024: 65); 16384
+    tokens, d 2048 46.2 / 47.3 / 36.3 (512); at 1.3 to 1.8 rounds a third slower)."""
+    segs = max(1, min(n_cu // -(-d // 256), _lib.MAX_EXPERTS))
+    return max(64, math.isqrt(T * d // 200) // 64 * 64, _ru(-(-T // segs), 64))
 
 
 class BwdWeights(NamedTuple):
@@ -129,15 +140,15 @@ def _stage(name):
 _INDEX_CACHE: dict = {}
 
 
-def _index_tensors(T: int, k: int, dev):
-    """Small constant index tensors of a backward of T tokens (cached per shape and
+def _index_tensors(T: int, k: int, dev, d: int):
+    """Small constant index tensors of a backward of T tokens of width d (cached per shape and
     device, so that a step makes no host-to-device copies): the one-segment offsets
     [0, T], the split-K token segments of the router weight gradient, the unit
     weights and the router-row column of the dx gather."""
-    key = (T, k, str(dev))
+    key = (T, k, str(dev), d)
     hit = _INDEX_CACHE.get(key)
     if hit is None:
-        split = max(WG_SPLIT, _ru(-(-T // _lib.MAX_EXPERTS), 64))  # at most MAX_EXPERTS segments
+        split = router_wgrad_rows(T, d, torch.cuda.get_device_properties(dev).multi_processor_count)
         nseg = max(1, -(-T // split))
         segs = torch.clamp(torch.arange(nseg + 1, dtype=torch.int64) * split, max=T).to(torch.int32).to(dev)
         one_seg = torch.tensor([0, T], dtype=torch.int32).to(dev)
@@ -236,7 +247,7 @@ def _router_core(x2d, hidden, w_out, bw: BwdWeights, dl, dx_rows, need_weights):
     E = dl.shape[1]
     dev = x2d.device
     s = ops._stream(x2d)
-    one_seg, segs, nseg, _, _ = _index_tensors(T, 1, dev)
+    one_seg, segs, nseg, _, _ = _index_tensors(T, 1, dev, d)
     with _stage("bwd_router"):
         da = torch.empty(T, _lib.ROUTER_HIDDEN, device=dev, dtype=_BF16)
         wdt = w_out.dtype
@@ -252,7 +263,7 @@ def _router_core(x2d, hidden, w_out, bw: BwdWeights, dl, dx_rows, need_weights):
     if not need_weights:
         return None, dw_out
     # dW_in = da^T x: a 128 x d output (few tiles) over K = T, split into token
-    # segments of WG_SPLIT rows whose fp32 partial sums are then reduced in order
+    # segments whose fp32 partial sums are then reduced in order
     dw_in = torch.empty(_lib.ROUTER_HIDDEN, d, device=dev, dtype=_BF16)
     with _stage("bwd_wgrad_router"):
         part = torch.empty(nseg, _lib.ROUTER_HIDDEN, d, device=dev, dtype=torch.float32)
@@ -332,7 +343,7 @@ def moe_backward(sv: Saved, dy: torch.Tensor, grad_aux: Optional[torch.Tensor], 
     A = T * k
     disp = sv.disp
     dy = dy.reshape(T, d).to(_BF16).contiguous()
-    _, _, _, _, extra = _index_tensors(T, k, x2d.device)
+    _, _, _, _, extra = _index_tensors(T, k, x2d.device, d)
     # the router's dx contribution goes to rows [A, A + T) of dxp and one unit-weight
     # gather sums both per token
     dxp, _, dw_in, dw_out, dyperm, dgu = _token_choice_core(sv, dy, grad_aux, w_out, bw, E, F, w_lb, w_z,

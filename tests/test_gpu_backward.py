@@ -351,3 +351,22 @@ def test_router_mlp_bwd(dev, E, T):
     assert _rel(outs[0][0], a64.grad) <= 4e-3
     assert _rel(outs[0][1], dl.double().cpu().t() @ s.detach()) <= 1e-5
     assert all(torch.equal(x, y) for x, y in zip(*outs))
+
+
+@pytest.mark.parametrize("T,d", [(1, 64), (65, 4096), (4097, 64), (3000, 2048), (8192, 8192), (70001, 256)])
+def test_router_weight_grads(dev, T, d):
+    """dW_in (its token segments of every length, a ragged last one) and dW_out against fp64 of
+    the same operands (bar 1e-2 rel-L2: da and dW_in are rounded to bf16 once each)."""
+    from kmoe import backward as BW
+
+    E = 4
+    g = torch.Generator(device=dev).manual_seed(T)
+    dl, a = (torch.randn(T, n, generator=g, device=dev) for n in (E, 128))
+    w = torch.randn(E, 128, generator=g, device=dev).to(torch.bfloat16)
+    x = torch.randn(T, d, generator=g, device=dev).to(torch.bfloat16)
+    dw_in, dw_out = BW.router_weight_grads(x, a, w, dl)
+    a64 = a.double().requires_grad_(True)
+    s = torch.nn.functional.silu(a64)
+    (s @ w.double().t()).backward(dl.double())
+    assert _rel(dw_in, a64.grad.t() @ x.double()) <= 1e-2
+    assert _rel(dw_out, dl.double().t() @ s.detach()) <= 1e-2

@@ -126,3 +126,17 @@ def test_ffn_block_keys_and_norm():
     assert kmoe.MoEFFNBlock(cfg, 0, ffn=m).ffn is m
     with pytest.raises(ValueError):
         blk.eval()(x.float())  # the fused path refuses CPU tensors
+
+
+def test_router_weight_gradient_segments():
+    """Token segments of the router's weight gradient: whole K-steps, at most MAX_EXPERTS of
+    them, and no more workgroups (segments times 256-column tiles) than CUs (8192 tokens, d
+    8192: 64 segments took twice the time of 16)."""
+    from kmoe import _lib, backward as BW
+
+    for T in (1, 64, 513, 2048, 4096, 8192, 16384, 65536, 1 << 20):
+        for d in (64, 256, 1024, 1536, 2048, 4096, 8192, 1 << 17):
+            rows = BW.router_wgrad_rows(T, d, 256)
+            n, tiles = -(-T // rows), -(-d // 256)
+            assert rows % 64 == 0 and rows >= 64 and 1 <= n <= _lib.MAX_EXPERTS
+            assert n == 1 or n * tiles <= 256, (T, d)
