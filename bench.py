@@ -5,9 +5,9 @@ python bench.py [--gpus 1] [--steps K] [--warmup W] [--config 2] [--no-cpu] [--n
 A step is one MoE-layer forward (router, dispatch, grouped SwiGLU GEMMs,
 combine, aux losses; train mode so the aux loss is computed) over one batch of
 synthetic input already resident in HBM.  Rank 0 prints one JSON line with
-whole-job tokens/s (timed with nothing but the forwards on the stream, plus a HIP
-event pair around the gate/up grouped GEMM on every EVENT_EVERY-th forward: the
-roofline of that dominant kernel), per-stage figures from a separate pass
+whole-job tokens/s (timed with nothing but the forwards on the stream), the roofline of
+the gate/up grouped GEMM, the dominant kernel, from HIP event pairs on every
+EVENT_EVERY-th of as many forwards right after, per-stage figures from a separate pass
 and a CPU baseline (the op-for-op torch-CPU port of the reference path, timed on this
 host on a bounded token sample).  Token-choice bf16 configs also report a
 "training" object: the training forward + backward step on the HIP kernels,
@@ -31,7 +31,7 @@ METRIC = "MoE-layer fwd tokens/sec (d2048,16e,top-2,bf16); % MFMA peak; dispatch
 PEAK_BF16 = 2.5e15
 PEAK_FP8 = 5.0e15
 PEAK_HBM = 8.0e12
-EVENT_EVERY = 5  # timed forwards per sampled gate/up event pair
+EVENT_EVERY = 5  # forwards per sampled gate/up event pair
 NEAR_TIE = 2.0 ** -16  # router logit gap counted as a near-tie
 
 
@@ -82,6 +82,34 @@ def stage_bytes_flops(wl, layer, fwd_state):
         "combine": ("byte", a_kept * d * s + T * d * s + 8.0 * a_all),
         "router": ("byte", t_in * d * s + t_in * E * 4 + t_in * k * 12),
     }
+
+
+def time_forwards(step, steps, sync):
+    """Seconds of the timed region: `steps` back-to-back forwards and nothing else (no stage
+    recorder, with which a layer runs its separate launches and not its one native call)."""
+    sync()
+    t0 = time.perf_counter()
+    for _ in range(steps):
+        step()
+    sync()
+    return time.perf_counter() - t0
+
+
+def sample_gate_up(step, steps, sync):
+    """Gate/up event pairs of every EVENT_EVERY-th of `steps` forwards, run right behind the
+    timed region at its clock (an event pair costs ~6 us of drain per event on this GPU, so it
+    is sampled rather than put on every forward)."""
+    from kmoe import ops
+
+    events = []
+    try:
+        for i in range(steps):
+            ops.set_stage_timing(events if i % EVENT_EVERY == 0 else None, only={"gemm_gate_up"})
+            step()
+        sync()
+    finally:
+        ops.set_stage_timing(None)
+    return events
 
 
 def run_gpu(args, wl, light=False):
@@ -147,19 +175,8 @@ def run_gpu(args, wl, light=False):
                 step()
             settle += 10
             torch.cuda.synchronize()
-        # timed region: K back-to-back forwards; the only extra work on the stream is
-        # a HIP event pair around the gate/up GEMM launch (the roofline kernel) on
-        # every EVENT_EVERY-th forward (an event pair costs ~6 us of drain per event
-        # on this GPU, so it is sampled rather than put on every forward)
-        timed = []
-        torch.cuda.synchronize()
-        t0 = time.perf_counter()
-        for i in range(args.steps):
-            ops.set_stage_timing(timed if i % EVENT_EVERY == 0 else None, only={"gemm_gate_up"})
-            step()
-        torch.cuda.synchronize()
-        t1 = time.perf_counter()
-        ops.set_stage_timing(None)
+        elapsed = time_forwards(step, args.steps, torch.cuda.synchronize)
+        timed = sample_gate_up(step, args.steps, torch.cuda.synchronize)
         # the materialising dispatch (tables + the row copy; what the fp8 path and
         # the C-ABI's xperm output use), outside the timed region, on this routing
         rows_us = None
@@ -208,7 +225,6 @@ def run_gpu(args, wl, light=False):
                 rec["GBps"] = round(amount / (us * 1e-6) / 1e9, 1)
                 rec["frac_hbm"] = round(amount / (us * 1e-6) / PEAK_HBM, 4)
         stage_out[name] = rec
-    elapsed = t1 - t0
     training = None
     if not light and not (wl.fp8 or wl.mod or wl.routing == "expert_choice") and not args.no_train:
         training = run_training(args, wl, layer, x)
@@ -306,7 +322,8 @@ def run_block(args, wl, layer, x):
             "unfused_tokens_per_s": round(wl.T / (ms["unfused"] * 1e-3), 1),
             "saved_us": round((ms["unfused"] - ms["fused"]) * 1e3, 1), "steps": steps,
             "fused_stages_us": stages, "training": training,
-            "note": "h + MoE(RMSNorm(h)), eval, bf16 norm weight; unfused = torch RMSNorm (embeddings.py:190-195) "
+            "note": "h + MoE(RMSNorm(h)), eval, bf16 norm weight; the stages are those of the separate launches (with "
+                    "a histogram launch in the dispatch), the timed pass is one native call; unfused = torch RMSNorm (embeddings.py:190-195) "
                     "+ kmoe layer + torch add"}
 
 
@@ -601,7 +618,7 @@ def main():
     tokens_per_s = wl.T * args.steps / res["elapsed"]
     flops_gu = res["work"]["gemm_gate_up"][1]
     peak = PEAK_FP8 if wl.fp8 else PEAK_BF16
-    us = res["gemm_us"]  # gate/up launch duration, HIP events inside the timed region
+    us = res["gemm_us"]  # gate/up launch duration, HIP events right behind the timed region
     achieved = flops_gu / (us * 1e-6) / 1e12
     traffic = load_traffic(f"gemm_gate_up_cfg{args.config}")
     out = {
