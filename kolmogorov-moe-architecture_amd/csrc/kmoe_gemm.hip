@@ -48,8 +48,7 @@ bool small_rows_product(bool gate_up, int E, int64_t max_rows, int64_t b_expert_
 int launch_gemm(bool gate_up, bool fp8, const void* A, const float* a_scale, const int32_t* row_token,
                 const int32_t* row_index, int64_t n_a_rows, const int32_t* offsets, int E, int K, int64_t max_rows,
                 const void* B, int64_t b_expert_rows, const float* b_scale, void* C, int64_t ldc, int n_valid,
-                int n_tiles, hipStream_t s, void* C2 = nullptr, void* gu_out = nullptr, int64_t ldb_bytes = 0,
-                const void* B2 = nullptr) {
+                int n_tiles, hipStream_t s, void* gu_out = nullptr, int64_t ldb_bytes = 0, const void* B2 = nullptr) {
   const int eb = fp8 ? 1 : 2;
   const int64_t slots = kmoe::ceil_div<int64_t>(max_rows, BM) + E;
   const int n_cu = kmoe::cu_count();
@@ -58,7 +57,7 @@ int launch_gemm(bool gate_up, bool fp8, const void* A, const float* a_scale, con
     kmoe::set_error("kmoe gemm: K bytes %d not a multiple of %d", kbytes, KB);
     return KMOE_ERR_SHAPE;
   }
-  GemmArgs g{};  // value-initialised: every optional output (C2, gu_out, Cf) starts null
+  GemmArgs g{};  // value-initialised: every optional output starts null
   g.A = static_cast<const uint8_t*>(A);
   g.lda_bytes = kbytes;
   g.a_scale = a_scale;
@@ -73,9 +72,7 @@ int launch_gemm(bool gate_up, bool fp8, const void* A, const float* a_scale, con
   g.C = static_cast<uint16_t*>(C);
   g.ldc = ldc;
   g.n_valid = n_valid;
-  g.C2 = static_cast<uint16_t*>(C2);
   g.gu_out = static_cast<uint16_t*>(gu_out);
-  g.Cf = nullptr;
   // every tile of the worst-case slot count, plus one narrow tile per resident
   // workgroup for the split tail
   int64_t blocks = slots * n_tiles + n_cu;
@@ -211,7 +208,7 @@ extern "C" int kmoe_gemm_gate_up_rows_gu(const void* x, const int32_t* row_index
   if (max_rows == 0) return KMOE_OK;
   const int Fp = round_up(F, 128);
   rc = launch_gemm(true, false, x, nullptr, row_token, row_index, n_x_rows, offsets, E, d, max_rows, w13_packed,
-                   2 * (int64_t)Fp, nullptr, h, Fp, Fp, Fp / 128, kmoe::as_stream(stream), nullptr, gu);
+                   2 * (int64_t)Fp, nullptr, h, Fp, Fp, Fp / 128, kmoe::as_stream(stream), gu);
   if (rc) return rc;
   return kmoe::check_launch("kmoe_gemm_gate_up_rows_gu");
 }
@@ -227,7 +224,7 @@ extern "C" int kmoe_gemm_gate_up_fp8_gu(const void* xperm, const float* xperm_sc
   if (max_rows == 0) return KMOE_OK;
   const int Fp = round_up(F, 128);
   rc = launch_gemm(true, true, xperm, xperm_scale, nullptr, nullptr, 0, offsets, E, d, max_rows, w13_packed,
-                   2 * (int64_t)Fp, w13_scale, h, Fp, Fp, Fp / 128, kmoe::as_stream(stream), nullptr, gu);
+                   2 * (int64_t)Fp, w13_scale, h, Fp, Fp, Fp / 128, kmoe::as_stream(stream), gu);
   if (rc) return rc;
   return kmoe::check_launch("kmoe_gemm_gate_up_fp8_gu");
 }
@@ -264,7 +261,7 @@ extern "C" int kmoe_gemm_grouped_weights(const void* a, const int32_t* offsets, 
   KMOE_REQUIRE(max_rows >= 0 && max_rows < ((int64_t)1 << 31), KMOE_ERR_SHAPE, "kmoe_gemm_grouped_weights: max_rows");
   if (max_rows == 0) return KMOE_OK;
   const int rc = launch_gemm(false, false, a, nullptr, nullptr, nullptr, 0, offsets, E, K, max_rows, b, N, nullptr, c,
-                             ldc, N, N / BN, kmoe::as_stream(stream), nullptr, nullptr, (int64_t)K * (b2 ? 1 : 2), b2);
+                             ldc, N, N / BN, kmoe::as_stream(stream), nullptr, (int64_t)K * (b2 ? 1 : 2), b2);
   if (rc) return rc;
   return kmoe::check_launch("kmoe_gemm_grouped_weights");
 }

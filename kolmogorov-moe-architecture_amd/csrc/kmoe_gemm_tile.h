@@ -150,26 +150,17 @@ struct Frag<true> {
   i32x8_t v;
 };
 
-// One MFMA operand fragment of K-substep `i` (bf16: 16 of K, chunk 2i+lh; fp8: 64
-// of K, chunks 4i+2lh and 4i+2lh+1) for LDS tile row `r`.
-template <bool FP8>
-__device__ __forceinline__ void read_frag(const uint8_t* l, int r, int i, int lh, Frag<FP8>& f) {
-  if constexpr (!FP8) {
-    f.v = *reinterpret_cast<const bf16x8_t*>(l + swz(r, 2 * i + lh));
-  } else {
-    const int ch = 4 * i + 2 * lh;
-    const i32x4_t lo = *reinterpret_cast<const i32x4_t*>(l + swz(r, ch));
-    const i32x4_t hi = *reinterpret_cast<const i32x4_t*>(l + swz(r, ch + 1));
-    f.v = i32x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-  }
+// One e4m3 MFMA operand fragment of K-substep `i` (64 of K, chunks 4i+2lh and 4i+2lh+1) for
+// LDS tile row `r`.
+__device__ __forceinline__ void read_frag(const uint8_t* l, int r, int i, int lh, Frag<true>& f) {
+  const int ch = 4 * i + 2 * lh;
+  const i32x4_t lo = *reinterpret_cast<const i32x4_t*>(l + swz(r, ch));
+  const i32x4_t hi = *reinterpret_cast<const i32x4_t*>(l + swz(r, ch + 1));
+  f.v = i32x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 }
 
-template <bool FP8>
-__device__ __forceinline__ void mfma(f32x16_t& acc, const Frag<FP8>& a, const Frag<FP8>& b) {
-  if constexpr (!FP8)
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, b.v, acc, 0, 0, 0);
-  else
-    acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a.v, b.v, acc, 0, 0, 0, 127, 0, 127);
+__device__ __forceinline__ void mfma(f32x16_t& acc, const Frag<true>& a, const Frag<true>& b) {
+  acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a.v, b.v, acc, 0, 0, 0, 127, 0, 127);
 }
 
 // bf16 tiles run on v_mfma_f32_16x16x32_bf16: on random data the 32x32x16 form holds the
@@ -350,9 +341,17 @@ __device__ __forceinline__ void store_staged(const uint8_t* lds, int tid, int m0
 // between C and C2 (the gate and up halves of a w13-ordered tile); fp32 to Cf.
 constexpr int OUT_BF16 = 0, OUT_SPLIT = 1, OUT_F32 = 2;
 
+// Four values as bf16.
+__device__ __forceinline__ i32x2_t pack4_bf16(float a, float b, float c, float d) {
+  const uint32_t lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));
+  const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{c, d}, bf16x2_t));
+  return i32x2_t{(int)lo, (int)hi};
+}
+
 // One output tile: rows [m0, min(m0 + 256, m_end)) of expert e against B rows of
 // full column tile nt (narrow part q when WNB < 4).
-// FP8: A/B bytes are e4m3; a_scale per A row, b_scale per B row (global row index).
+// FP8: A/B bytes are e4m3; a_scale per A row, b_scale per B row (global row index).  Narrow
+// tiles only (full ones: gemm_full_tiles), always with NMA = 4.
 // GATHER: A is the unpermuted activation matrix and permuted row r is its row
 // row_index[row_token[r]] (row_token[r] without row_index): the dispatch gather is
 // fused into the A loads.
@@ -364,12 +363,13 @@ constexpr int OUT_BF16 = 0, OUT_SPLIT = 1, OUT_F32 = 2;
 // run with NMA < 4 (the first NMA blocks), which skips the other blocks' fragment
 // reads, MFMAs and epilogue (their accumulators stay 0 and are never stored).  The
 // waves of a workgroup may differ in NMA: loads, LDS writes and barriers are the same.
-// DUAL: see dual_step.
+// DUAL: see dual_step_second.
 template <bool GATE_UP, bool FP8, bool GATHER, int WNB, bool SAVE_GU = false, bool RSCALE = false, int NMA = 4,
           bool DUAL = false>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, uint8_t* lds, int e, int m0, int m_end, int nt,
                                           int q) {
   static_assert(WNB == 4 || WNB == 2 || WNB == 1, "tile width");
+  static_assert(!FP8 || (WNB < 4 && NMA == 4 && !GATHER && !RSCALE && !DUAL), "e4m3 tiles here are narrow");
   // bf16: 16x16x32 MFMAs, 16-row A and B blocks (MA x NBB per wave, NAB of them holding
   // rows); fp8: 32x32x64, 32-row blocks
   constexpr bool M16 = !FP8;
@@ -482,29 +482,20 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, uint8_t* lds, int e
   };
   Frag<FP8> fa[2][MA], fb[2][NBB];
   const int r16 = lane & 15, lq = lane >> 4;
+  // e4m3: all fragments of K-substep i of stage st
   auto rd = [&](int st, int i, Frag<FP8> (&a)[MA], Frag<FP8> (&b)[NBB]) {
-    if constexpr (NMA > 0) {
-      const uint8_t* la = la_buf(st);
-      const uint8_t* lb = lb_buf(st);
-      if constexpr (M16) {
+    if constexpr (FP8) {
 #pragma unroll
-        for (int j = 0; j < NBB; ++j)
-          read_frag16(lb, b_lds_row<GATE_UP, WNB>(wn, j >> 1, 16 * (j & 1) + r16), i, lq, b[j]);
+      for (int mi = 0; mi < NMA; ++mi) read_frag(la_buf(st), wm * 128 + mi * 32 + lr, i, lh, a[mi]);
 #pragma unroll
-        for (int mi = 0; mi < NAB; ++mi) read_frag16(la, wm * 128 + mi * 16 + r16, i, lq, a[mi]);
-      } else {
-#pragma unroll
-        for (int mi = 0; mi < NMA; ++mi) read_frag<FP8>(la, wm * 128 + mi * 32 + lr, i, lh, a[mi]);
-#pragma unroll
-        for (int j = 0; j < WNB; ++j) read_frag<FP8>(lb, b_lds_row<GATE_UP, WNB>(wn, j, lr), i, lh, b[j]);
-      }
+      for (int j = 0; j < WNB; ++j) read_frag(lb_buf(st), b_lds_row<GATE_UP, WNB>(wn, j, lr), i, lh, b[j]);
     }
   };
   auto mma1 = [&](Acc& c, const Frag<FP8>& b, const Frag<FP8>& a) {
     if constexpr (M16)
       mfma16(c, b, a);
     else
-      mfma<FP8>(c, b, a);
+      mfma(c, b, a);
   };
   auto mma = [&](const Frag<FP8> (&a)[MA], const Frag<FP8> (&b)[NBB]) {
 #pragma unroll
@@ -524,14 +515,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, uint8_t* lds, int e
   // tile data.  Those blocks are written into stage (kt+1)%2 (which every wave
   // stopped reading at step kt-1's barrier) over the substeps, each block reloaded
   // with step kt+2's data right after its write, so a load has a whole step to land
-  // and the LDS write traffic is spread (bf16: about 6/5/5 sixteenths of the blocks
-  // in substeps 0-2; fp8: half in each substep).  In the last substep, after most of
+  // and the LDS write traffic is spread: half of the blocks in each of the two substeps.  In the last substep, after most of
   // its MFMAs, the wave waits for its LDS writes and reads, then one barrier publishes
   // stage kt+1, whose first fragments are read under the last few MFMAs.  Register
   // dependencies give the vmcnt waits; the scheduling groups interleave the LDS and
   // memory operations with the MFMAs, fragment reads first.
-  constexpr int RD = NMA > 0 ? (FP8 ? 2 : 1) * (NAB + NBB) : 0;  // LDS reads of a substep's fragments
-  constexpr int NMS = NAB * NBB;                                    // MFMAs per substep
+  constexpr int RD = 2 * (NAB + NBB);  // e4m3: LDS reads of a substep's fragments
+  constexpr int NMS = NAB * NBB;       // MFMAs per substep
   for (int qq = 0; qq < NBLK; ++qq) load_block(qq, 0);
   for (int qq = 0; qq < NBLK; ++qq) write_block(qq, 0);
   for (int qq = 0; qq < NBLK; ++qq) load_block(qq, 1);
@@ -658,22 +648,16 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, uint8_t* lds, int e
     }
   }
   auto step = [&](int kt, auto last_tag) {
-    if constexpr (M16) {
-      step16(kt, last_tag);
-      return;
-    }
+    if constexpr (M16) return step16(kt, last_tag);
     constexpr bool LAST = decltype(last_tag)::value;
     const int cur = kt & 1, nxt = cur ^ 1;
     static_for<0, NSUB>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
       constexpr int bi = i & 1;
-      // blocks [q0, q1) are written and reloaded in this substep.  bf16 (4 substeps):
-      // about 6/5/5 sixteenths in substeps 0-2.  fp8 (2 substeps): half in each, the
-      // last substep's before its barrier (all in substep 0 crowded the LDS queue with
-      // that substep's fragment reads: 3% slower).
-      constexpr int C1 = (NBLK * 6 + 8) / 16, C2 = (NBLK * 11 + 8) / 16;
-      constexpr int q0 = NSUB == 4 ? (i == 0 ? 0 : i == 1 ? C1 : i == 2 ? C2 : NBLK) : i * NBLK / NSUB;
-      constexpr int q1 = NSUB == 4 ? (i == 0 ? C1 : i == 1 ? C2 : NBLK) : (i + 1) * NBLK / NSUB;
+      // blocks [q0, q1) are written and reloaded in this substep: half in each, the last
+      // substep's before its barrier (all in substep 0 crowded the LDS queue with that
+      // substep's fragment reads: 3% slower)
+      constexpr int q0 = i * NBLK / NSUB, q1 = (i + 1) * NBLK / NSUB;
       constexpr int nq = LAST ? 0 : q1 - q0;
       constexpr bool RDN = i + 1 < NSUB || !LAST;
       // next substep's fragments first: they are on the MFMA critical path
@@ -752,29 +736,16 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, uint8_t* lds, int e
     for (int r = 0; r < 16; ++r)
       sbr[j][r] = FP8 ? sb_l[b_lds_row<GATE_UP, WNB>(wn, j, 8 * (r >> 2) + 4 * lh + (r & 3))] : 1.0f;
   float sar = 1.0f;
+  // e4m3: output r of block (mi, jo), descaled
   auto result = [&](int mi, int r, int jo) -> float {
     if (GATE_UP) {
       constexpr int UJ = GU1 ? 0 : WNB / 2, UR = GU1 ? 8 : 0;  // up value: block jo + UJ, run + UR/4
-      float gg = acc[mi][jo][r], u = acc[mi][jo + UJ][r + UR];
-      if (FP8) {
-        gg *= sar * sbr[jo][r];
-        u *= sar * sbr[jo + UJ][r + UR];
-      }
-      if (RSCALE) {
-        gg *= sar;
-        u *= sar;
-      }
+      const float gg = acc[mi][jo][r] * (sar * sbr[jo][r]);
+      const float u = acc[mi][jo + UJ][r + UR] * (sar * sbr[jo + UJ][r + UR]);
       return silu_fast_f32(gg) * u;
     } else {
-      float v = acc[mi][jo][r];
-      if (FP8) v *= sar * sbr[jo][r];
-      return v;
+      return acc[mi][jo][r] * (sar * sbr[jo][r]);
     }
-  };
-  auto pack4 = [](float a, float b, float c, float d) {
-    const uint32_t lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));
-    const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{c, d}, bf16x2_t));
-    return i32x2_t{(int)lo, (int)hi};
   };
   if constexpr (M16) {
     // 16x16 blocks: acc[mi][j][t] is output row wm*128 + mi*16 + l%16 against B row
@@ -801,22 +772,21 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, uint8_t* lds, int e
             v[t] = acc[mi][jo][t];
           }
         }
-        *reinterpret_cast<i32x2_t*>(wb16 + mi * 16 * OSTR + jo * 32) = pack4(v[0], v[1], v[2], v[3]);
+        *reinterpret_cast<i32x2_t*>(wb16 + mi * 16 * OSTR + jo * 32) = pack4_bf16(v[0], v[1], v[2], v[3]);
       }
     }
   } else {
     // lane's row of block 0 and its first column (c = 0) of output column block 0
     uint8_t* const wbase = lds + (wm * 128 + lr) * OSTR + (wn * (NC / 2) + 4 * lh) * 2;
 #pragma unroll
-    for (int mi = 0; mi < 4; ++mi) {
-      if (mi >= NMA) break;  // rows past the expert's end: never stored
-      if constexpr (FP8 || RSCALE) sar = sa_l[wm * 128 + mi * 32 + lr];
+    for (int mi = 0; mi < NMA; ++mi) {
+      sar = sa_l[wm * 128 + mi * 32 + lr];
 #pragma unroll
       for (int jo = 0; jo < NJ; ++jo)
 #pragma unroll
         for (int c = 0; c < NCR; ++c)
           *reinterpret_cast<i32x2_t*>(wbase + mi * 32 * OSTR + (jo * 32 + 8 * c) * 2) =
-              pack4(result(mi, 4 * c, jo), result(mi, 4 * c + 1, jo), result(mi, 4 * c + 2, jo),
+              pack4_bf16(result(mi, 4 * c, jo), result(mi, 4 * c + 1, jo), result(mi, 4 * c + 2, jo),
                     result(mi, 4 * c + 3, jo));
     }
   }
@@ -840,22 +810,21 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, uint8_t* lds, int e
         for (int j = 0; j < NBB; ++j) {
           const int col = b_lds_row<true, WNB>(wn, j >> 1, 16 * (j & 1));
           *reinterpret_cast<i32x2_t*>(wb2 + mi * 16 * OSTR2 + col * 2) =
-              pack4(acc[mi][j][0], acc[mi][j][1], acc[mi][j][2], acc[mi][j][3]);
+              pack4_bf16(acc[mi][j][0], acc[mi][j][1], acc[mi][j][2], acc[mi][j][3]);
         }
     } else {
       uint8_t* const wb2 = lds + (wm * 128 + lr) * OSTR2 + 4 * lh * 2;
 #pragma unroll
-      for (int mi = 0; mi < 4; ++mi) {
-        if (mi >= NMA) break;
-        if constexpr (FP8) sar = sa_l[wm * 128 + mi * 32 + lr];
+      for (int mi = 0; mi < NMA; ++mi) {
+        sar = sa_l[wm * 128 + mi * 32 + lr];
 #pragma unroll
         for (int j = 0; j < WNB; ++j) {
           const int col = b_lds_row<true, WNB>(wn, j, 0);
-          auto gv = [&](int r) { return FP8 ? acc[mi][j][r] * (sar * sbr[j][r]) : acc[mi][j][r]; };
+          auto gv = [&](int r) { return acc[mi][j][r] * (sar * sbr[j][r]); };
 #pragma unroll
           for (int c = 0; c < 4; ++c)
             *reinterpret_cast<i32x2_t*>(wb2 + mi * 32 * OSTR2 + (col + 8 * c) * 2) =
-                pack4(gv(4 * c), gv(4 * c + 1), gv(4 * c + 2), gv(4 * c + 3));
+                pack4_bf16(gv(4 * c), gv(4 * c + 1), gv(4 * c + 2), gv(4 * c + 3));
         }
       }
     }
@@ -877,12 +846,6 @@ __device__ __forceinline__ i32x4_t merge32(i32x2_t x, i32x2_t y) {
   const auto b = __builtin_amdgcn_permlane32_swap((unsigned)x[1], (unsigned)y[1], false, false);
   return i32x4_t{(int)a[0], (int)b[0], (int)a[1], (int)b[1]};
 }
-__device__ __forceinline__ i32x2_t pack4_bf16(float a, float b, float c, float d) {
-  const uint32_t lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));
-  const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{c, d}, bf16x2_t));
-  return i32x2_t{(int)lo, (int)hi};
-}
-
 // LDS of the full-tile loop behind its stages: the experts' slot table (lo, hi, inclusive
 // slot count of each) and two sets of A-row and B-row scales.
 constexpr int FT_SLOTS = NST * 2 * TB;
@@ -1021,9 +984,9 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
     constexpr int NMA = decltype(nma_tag)::value;
     if constexpr (NMA > 0) {
 #pragma unroll
-      for (int mi = 0; mi < NMA; ++mi) read_frag<true>(la_buf(s), wm * 128 + mi * 32 + lr, i, lh, a[mi]);
+      for (int mi = 0; mi < NMA; ++mi) read_frag(la_buf(s), wm * 128 + mi * 32 + lr, i, lh, a[mi]);
 #pragma unroll
-      for (int j = 0; j < NBB; ++j) read_frag<true>(lb_buf(s), b_lds_row<GATE_UP, 4>(wn, j, lr), i, lh, b[j]);
+      for (int j = 0; j < NBB; ++j) read_frag(lb_buf(s), b_lds_row<GATE_UP, 4>(wn, j, lr), i, lh, b[j]);
     }
   };
 
@@ -1046,7 +1009,7 @@ __device__ __forceinline__ void gemm_full_tiles(const GemmArgs& g, uint8_t* lds,
     auto mma_part = [&](const Frag<true> (&a)[MA], const Frag<true> (&b)[NBB], auto lo_tag, auto hi_tag) {
       static_for<decltype(lo_tag)::value, decltype(hi_tag)::value>([&](auto xc) {
         constexpr int x = decltype(xc)::value;
-        mfma<true>(acc[x / NBB][x % NBB], b[x % NBB], a[x / NBB]);
+        mfma(acc[x / NBB][x % NBB], b[x % NBB], a[x / NBB]);
       });
     };
     static_for<0, NSUB>([&](auto ic) {
