@@ -709,16 +709,17 @@ def test_mod_select_parity(dev, B, S, keep, ties):
     assert np.array_equal(out.out_map.cpu().numpy(), om)
 
 
-# ------------------------------------------------------------------ full-tile loop
+# ------------------------------------------------------------------ full tiles
 @pytest.mark.parametrize("path,d", [("rows", 64), ("rows", 128), ("rows", 192), ("rows", 320), ("rscale", 128),
                                     ("rscale", 256), ("save_gu", 128), ("save_gu", 192), ("fp8", 128), ("fp8", 256),
                                     ("fp8", 384)])
 def test_full_tile_loop(dev, path, d):
-    """Several full tiles per workgroup (more than two tiles per CU) with one, two, three
-    and more K-steps (d 64 per step, fp8 128), experts of 0, 1, 33, 64, 65 and many rows:
-    the gate/up product against fp32 matmuls of the same operands (fp8: the dequantised
-    ones).  A wrong stage, row lookup or scale set of a following tile gives an error of
-    order 1; rounding h to bf16 gives 2^-9 at most per value (bar 4e-3 rel-L2)."""
+    """Nearly two rounds of tiles (bf16: one workgroup each; e4m3 of two and three K-steps: in
+    the loop; of one: narrow ones) with one, two, three and more K-steps (d 64 per step, fp8
+    128), experts of 0, 1, 33, 64, 65 and many rows: the gate/up product against fp32 matmuls
+    of the same operands (fp8: the dequantised ones).  A wrong stage, row lookup or scale set
+    gives an error of order 1; rounding h to bf16 gives 2^-9 at most per value (bar 4e-3
+    rel-L2).  test_fp8_full_tile_loop has more tiles per workgroup."""
     F = 256
     n_cu = torch.cuda.get_device_properties(dev).multi_processor_count
     counts = [1, 0, 33, 64, 65, 256, 256 * (n_cu // 3) + 17, 256 * (n_cu // 2) + 129]
@@ -757,6 +758,59 @@ def test_full_tile_loop(dev, path, d):
         if gu is not None:
             packed = torch.cat([gg[:, :128], uu[:, :128], gg[:, 128:], uu[:, 128:]], 1)
             assert rel(gu[s:t], packed) <= 4e-3, (path, d, e, counts[e])
+
+
+@pytest.mark.parametrize("path", ["gate_up", "save_gu", "down"])
+@pytest.mark.parametrize("K", [256, 384, 512])
+def test_fp8_full_tile_loop(dev, path, K):
+    """Four and more e4m3 tiles per workgroup of the full-tile loop with two (the extra barrier
+    before the scale set of the next tile), three (the stages swap between tiles) and four
+    K-steps, experts of 0 to 65 and many rows, so that tiles with and without waves to skip
+    follow each other: gate/up, with saved pre-activations, and down against fp32 products of
+    the decoded operands (bar 4e-3 rel-L2: one bf16 rounding; a wrong stage, tile or scale set
+    gives an error of order 1)."""
+    n_cu = torch.cuda.get_device_properties(dev).multi_processor_count
+    N = 768 if path != "down" else 1536  # six column tiles a slot
+    half = 256 * (n_cu // 3)
+    counts = [half + 17, 1, 0, 33, 64, 65, 256, half + 129, 31, half // 4 + 200]
+    E, A = len(counts), sum(counts)
+    tiles = 6 * sum(-(-c // 256) for c in counts)
+    assert tiles >= 4 * n_cu
+    off_l = np.concatenate([[0], np.cumsum(counts)])
+    off = torch.tensor(off_l, dtype=torch.int32, device=dev)
+    g = torch.Generator(device=dev).manual_seed(K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    a, a_s = ops.quant_rows_fp8(bf16(rnd(A, K)))
+    av = a.view(torch.float8_e4m3fn).float() * a_s[:, None]
+    rel = lambda x, y: float((x.float() - y).norm() / y.norm())
+    if path == "down":
+        d, F = N, K
+    else:
+        d, F = K, N
+    w1, w2, w3 = (bf16(rnd(*s) * s[1] ** -0.5) for s in ((E, d, F), (E, d, F), (E, F, d)))
+    pw = ops.pack_weights(w1, w2, w3, fp8=True)
+    w1, w2, w3 = (ops.fake_quant_cols_e4m3(w).float() for w in (w1, w2, w3))
+    gu = None
+    if path == "down":
+        out = ops.gemm_down(a, a_s, off, pw, A)
+    elif path == "save_gu":
+        out, gu = ops.gemm_gate_up(a, a_s, off, pw, A, save_gu=True)
+    else:
+        out = ops.gemm_gate_up(a, a_s, off, pw, A)
+    for e in range(E):
+        s, t = int(off_l[e]), int(off_l[e + 1])
+        if s == t:
+            continue
+        # whole experts and, of the long ones, their first and last tiles alone
+        for lo, hi in {(s, t), (s, min(t, s + 256)), (max(s, t - 256), t)}:
+            if path == "down":
+                assert rel(out[lo:hi], av[lo:hi] @ w3[e]) <= 4e-3, (e, lo, hi)
+                continue
+            gg, uu = av[lo:hi] @ w1[e], av[lo:hi] @ w2[e]
+            assert rel(out[lo:hi], torch.nn.functional.silu(gg) * uu) <= 4e-3, (e, lo, hi)
+            if gu is not None:
+                packed = torch.stack([gg.view(-1, F // 128, 128), uu.view(-1, F // 128, 128)], 2).reshape(hi - lo, 2 * F)
+                assert rel(gu[lo:hi], packed) <= 4e-3, (e, lo, hi)
 
 
 @pytest.mark.parametrize("d", [128, 256, 384])
