@@ -3,9 +3,11 @@
 // There every expert's weights are read once for a handful of rows, so the product is bound
 // by streaming the packed weights (a plain read of this size reaches 6.1 TB/s).  The
 // 256-row tiles of kmoe_gemm_tile.h stream them through LDS, one workgroup per CU; here
-// each wave loads its weight rows straight into MFMA operand registers, at five
-// workgroups per CU: 48 tokens, top-2 of 16 experts, d 2048, F 2816: gate/up 77.6 -> 68.0
-// us (5.4 TB/s), down 44.3 -> 37.8; 1 token 23.9 -> 13.0 and 26.2 -> 9.3 us.
+// each wave loads its weight rows straight into MFMA operand registers, at four
+// workgroups per CU (104 to 122 registers a lane).  d 2048, F 2816, 16 experts, top-2, weights
+// not in a cache, 256-row tiles -> here: 96 rows, 6 an expert, gate/up 77.0 -> 66.1 us (5.6
+// TB/s), down 39.7 -> 35.6 (5.2); one token, two experts, 21.5 -> 12.2 (3.8) and 25.9 -> 8.8
+// (2.6), bound by latency.
 //
 // Operand fragments (v_mfma_f32_16x16x32_bf16, weights first): lane l holds row l % 16 of a
 // 16-row block at the 8 K values of chunk l / 16, so one load instruction takes 64
@@ -83,8 +85,8 @@ __device__ __forceinline__ void put_gate_up(const GemmArgs& g, int row, int f, f
 // weights' K range to itself, so nothing is shared until the four partial sums are added
 // in wave order through LDS.
 // Two K-steps in flight per wave: more, at fewer waves per CU, stream slower (gate/up of 96
-// rows over 16 experts, d 2048, F 2816: 1 step 67.1 us, 2 67.6, 3 73.2, 4 75.7, 8 97.0; the
-// 256-row tiles 84.5).  Interleaving the waves' steps, eight waves per workgroup and
+// rows over 16 experts, d 2048, F 2816, in one run: 1 step 67.1 us, 2 67.6, 3 73.2, 4 75.7, 8
+// 97.0).  Interleaving the waves' steps, eight waves per workgroup and
 // non-temporal weight loads were slower too.
 constexpr int DEPTH = 2;
 template <bool GATE_UP, bool GATHER, bool SAVE_GU, bool RSCALE, bool DUAL>

@@ -859,8 +859,8 @@ static_assert(FT_LDS <= GEMM_LDS, "LDS of the full-tile loop");
 // starts with its first stage in LDS and its second step in flight, and the epilogue
 // stores straight from registers.  One workgroup fills a CU (128 KiB of stages, 512
 // registers), so whatever runs between two tiles leaves its matrix cores idle, and an
-// e4m3 tile has half the K-steps of a bf16 one: the layer of 8192 tokens (6144 kept), d
-// 2048, F 2816 375 -> 358 us against one workgroup per tile.  (bf16 tiles the same way: 1045
+// e4m3 tile has half the K-steps of a bf16 one: 12288 rows over 16 experts, d 2048, F
+// 2816, gate/up + down 216 -> 197 us against one workgroup per tile.  (bf16 tiles the same way: 1045
 // -> 1025 us at 16384 tokens, eleven rounds, but 2% slower at one to three rounds; they
 // stay one workgroup per tile.)  For products with full_tile_loop().
 // NMA (4, 2, 1 or 0, per tile and wave): the wave's 32-row blocks that hold rows of the
