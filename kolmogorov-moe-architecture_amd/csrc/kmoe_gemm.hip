@@ -17,18 +17,21 @@ int64_t small_slots(int E, int64_t max_rows) { return std::min<int64_t>(max_rows
 // - where its grid is at most two workgroups per CU, as latency then counts: d 256, F 352, 4
 //   experts: 128 tokens 10.0 / 15.9, 512 tokens 15.9 / 16.3 (down 6.3 / 8.2 at 288
 //   workgroups, gate/up 9.6 / 8.2 at 864);
-// - and at up to 8 rows per expert (max_rows / E), where the weights are the traffic and are
-//   read once.  Gate/up and down at 4, 8, 10 and 16 rows each: 16 experts, d 2048, F 2816: 66
-//   / 81 and 36 / 43, 70 / 81 and 38 / 43, 72 / 81 and 40 / 43, 79 / 77 and 42 / 40; 64
-//   experts, d 2048, F 1408: 125 / 134 and 65 / 69, 134 / 135 and 69 / 69, 140 / 135 and 71 /
-//   70, 159 / 136 and 81 / 70; 8 experts, d 2048, F 2816: 37 / 40 and 20 / 33, 38 / 39 and 21
-//   / 33, 39 / 37 and 20 / 32, 43 / 38 and 22 / 32;
+// - and at few rows per expert (max_rows / E), where the weights are the traffic and are read
+//   once: up to 6 where one tile per expert and column tile fills the CUs in whole rounds or
+//   in more than two, else up to 10.  Gate/up and down at 4, 8 and 10 rows each: 64 experts, d
+//   2048, F 1408 (704 and 512 tiles) 125 / 134 and 65 / 69, 134 / 135 and 69 / 69, 140 / 135
+//   and 71 / 70; 32 experts, d 2048, F 768 (192 and 256) 38.6 / 41.3 and 25.5 / 23.2, 38.7 /
+//   39.4 and 25.6 / 22.8; 16 experts, d 2048, F 2816 (352 and 128) 66 / 81 and 36 / 43, 70 / 81
+//   and 38 / 43, 72 / 81 and 40 / 43; 8 experts, d 2048, F 2816 (176 and 64) 37 / 40 and 20 /
+//   33, 38 / 39 and 21 / 33, 39 / 37 and 20 / 32.  At 16 rows: 159 / 136 and 81 / 70 (64
+//   experts), 79 / 77 and 42 / 40 (16), 43 / 38 and 22 / 32 (8);
 // - if not too many workgroups stream one expert's weights again for its further slots: at
-//   most three per CU over the slots that the rows can fill.  All rows on one expert, gate/up
-//   and down: 16 experts, 64 rows (352 workgroups in gate/up) 18 / 21 and 13 / 26, 128 rows
-//   (704) 26 / 21 and 13 / 26, 160 rows (880) 33 / 21 and 23 / 26; 64 experts, 256 rows (704)
-//   26 / 21 and 15 / 15, 640 rows (1760) 56 / 22 and 31 / 16.  (Zipf 1.2 routing at up to 8
-//   rows per expert: 0.75 to 1.06 in gate/up, 0.7 to 1.0 in down.)
+//   most three per CU over the full slots that the rows can make.  All rows on one expert,
+//   gate/up and down: 16 experts, 64 rows (352 workgroups in gate/up) 18 / 21 and 13 / 26, 128
+//   rows (704) 26 / 21 and 13 / 26, 160 rows (880) 33 / 21 and 23 / 26; 64 experts, 256 rows
+//   (704) 26 / 21 and 15 / 15, 640 rows (1760) 56 / 22 and 31 / 16.  (Zipf 1.2 routing: 0.75
+//   to 1.08 of the tiles' time in gate/up, 0.7 to 1.06 in down.)
 // (A kernel of 128-row slots for 10 to 64 rows per expert, weights to registers and rows
 // through LDS, measured 4% faster alone at 16 to 32 rows and 2% slower inside a layer.)
 bool small_rows_product(bool gate_up, int E, int64_t max_rows, int64_t b_expert_rows, int64_t ldb_bytes,
@@ -38,8 +41,10 @@ bool small_rows_product(bool gate_up, int E, int64_t max_rows, int64_t b_expert_
   const int64_t n_ct = (int64_t)n_tiles * (gate_up ? BN / 2 : BN) / small_cols(gate_up);
   const int64_t n_cu = kmoe::cu_count();
   if (small_slots(E, max_rows) * n_ct <= 2 * n_cu) return true;
+  const int64_t tiles = (int64_t)E * n_tiles;
+  const int rows = tiles % n_cu == 0 || tiles > 2 * n_cu ? 6 : 10;
   // (a launch takes 2^24 workgroups of 256)
-  return max_rows <= 8 * (int64_t)E && max_rows / SMALL_ROWS * n_ct <= 3 * n_cu &&
+  return max_rows <= rows * (int64_t)E && max_rows / SMALL_ROWS * n_ct <= 3 * n_cu &&
          small_slots(E, max_rows) * n_ct < 1 << 24;
 }
 
