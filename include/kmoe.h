@@ -461,7 +461,8 @@ int kmoe_rmsnorm_bwd(const void* dn, const void* x, int x_dtype, const void* wei
 
 /* Router MLP backward: da = (dl . w_out) * silu'(a) -> (T, 128) bf16 and
  * dw_out = dl^T silu(a) -> (E, 128) (bf16 or f32), reduced in a fixed order.
- * hidden_pre: a from kmoe_router_train.  workspace: kmoe_router_bwd_workspace_bytes.
+ * hidden_pre: a from kmoe_router_train.  workspace: kmoe_router_bwd_workspace_bytes (asked
+ * for on the device of the call: at most three partial sums per CU).
  * dw_in = da^T x and dx += da . w_in follow with kmoe_gemm_wgrad_rows / kmoe_gemm_grouped
  * (w_in^T packed by kmoe_pack_w_in_t).                                       */
 size_t kmoe_router_bwd_workspace_bytes(int64_t T, int E);
